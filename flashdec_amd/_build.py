@@ -37,6 +37,7 @@ ARCH = "gfx950"
 SOURCES = {
     "capi.hip": [],
     "paged_decode.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
+    "even_decode.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=16"],
     "rope_append.hip": ["-ffp-contract=off", "-mllvm", "-amdgpu-kernarg-preload-count=16"],
 }
 

@@ -17,6 +17,7 @@ LIB_NAME = "libflashdec_hip.so"
 LIB_PATH = Path(__file__).resolve().with_name(LIB_NAME)
 
 FD_OK = 0
+FD_E_UNSUPPORTED = -2
 FD_DTYPE_F16 = 0
 FD_DTYPE_BF16 = 1
 FD_DTYPE_F32 = 2
@@ -130,6 +131,9 @@ EXPORTED_SYMBOLS = (
     "fd_paged_decode_noalloc",
     "fd_paged_decode_noalloc_prepare",
     "fd_paged_decode_cascade",
+    "fd_paged_decode_even",
+    "fd_paged_decode_even_floats",
+    "fd_paged_decode_even_pays",
     "fd_paged_decode_plan",
     "fd_paged_decode_balance_target",
     "fd_fused_rope_kv_append",
@@ -175,6 +179,12 @@ def load_library():
         lib.fd_paged_decode_noalloc_prepare.restype = ctypes.c_int
         lib.fd_paged_decode_cascade.argtypes = [ctypes.POINTER(PagedDecodeArgs), ctypes.POINTER(CascadeArgs), _vp]
         lib.fd_paged_decode_cascade.restype = ctypes.c_int
+        lib.fd_paged_decode_even.argtypes = [ctypes.POINTER(PagedDecodeArgs), _vp, _i64, _vp]
+        lib.fd_paged_decode_even.restype = ctypes.c_int
+        lib.fd_paged_decode_even_floats.argtypes = [ctypes.POINTER(PagedDecodeArgs)]
+        lib.fd_paged_decode_even_floats.restype = ctypes.c_int
+        lib.fd_paged_decode_even_pays.argtypes = [ctypes.POINTER(PagedDecodeArgs)]
+        lib.fd_paged_decode_even_pays.restype = ctypes.c_int
         lib.fd_paged_decode_balance_target.argtypes = [_i64, _i64]
         lib.fd_paged_decode_balance_target.restype = ctypes.c_int
         lib.fd_paged_decode_plan.argtypes = [_i64, _i64, _i64, _i64, _i64, _i64]
@@ -282,6 +292,29 @@ def paged_decode_cascade(args: PagedDecodeArgs, cascade: CascadeArgs, stream: in
     args.struct_size = ctypes.sizeof(PagedDecodeArgs)
     cascade.struct_size = ctypes.sizeof(CascadeArgs)
     check(lib.fd_paged_decode_cascade(ctypes.byref(args), ctypes.byref(cascade), stream), "fd_paged_decode_cascade")
+
+
+def paged_decode_even(args: PagedDecodeArgs, workspace: int, floats: int, stream: int) -> bool:
+    """``fd_paged_decode_even``: the batch's tokens in equal shares; ``workspace`` a device pointer.
+    False where these pointers' alignment needs ``paged_decode`` (nothing was launched)."""
+    lib = load_library()
+    args.struct_size = ctypes.sizeof(PagedDecodeArgs)
+    rc = lib.fd_paged_decode_even(ctypes.byref(args), workspace, floats, stream)
+    if rc == FD_E_UNSUPPORTED:
+        return False
+    check(rc, "fd_paged_decode_even")
+    return True
+
+
+def paged_decode_even_floats(args: PagedDecodeArgs) -> int:
+    """fp32 words of workspace that ``paged_decode_even`` needs for this call where the library would
+    take it, else 0."""
+    lib = load_library()
+    args.struct_size = ctypes.sizeof(PagedDecodeArgs)
+    pays = lib.fd_paged_decode_even_pays(ctypes.byref(args))
+    if pays < 0:
+        check(pays, "fd_paged_decode_even_pays")
+    return lib.fd_paged_decode_even_floats(ctypes.byref(args)) if pays else 0
 
 
 def paged_decode_plan(num_seqs, num_q_heads, num_kv_heads, head_dim, max_seq_len, total_seq_len=0) -> int:

@@ -191,22 +191,29 @@ class _SplitWorkspace:
 _WORKSPACES = {}
 
 
-def _auto_workspace(q, num_kv_heads, num_splits, stream):
-    num_seqs, num_q_heads, head_dim = q.shape
-    floats = num_seqs * num_q_heads * num_splits * (head_dim + 2)
-    counters = num_seqs * num_kv_heads * _lib.SPLIT_COUNTER_STRIDE
-    key = (q.device.index, stream)
+def _stream_workspace(device, floats, counters, stream):
+    """This stream's workspace, grown to the sizes asked for; a private one inside a graph capture
+    that it is too small for."""
+    key = (device.index, stream)
     ws = _WORKSPACES.get(key)
     if ws is None or ws.flat.numel() < floats or ws.counters.numel() < counters:
         if torch.cuda.is_current_stream_capturing():
-            return _SplitWorkspace(q.device, floats, counters).views(num_seqs, num_q_heads, num_splits, head_dim)
+            return _SplitWorkspace(device, floats, counters)
         grow = 1 if ws is None else 2
         ws = _SplitWorkspace(
-            q.device,
+            device,
             max(floats, grow * (ws.flat.numel() if ws else 0)),
             max(counters, grow * (ws.counters.numel() if ws else 0)),
         )
         _WORKSPACES[key] = ws
+    return ws
+
+
+def _auto_workspace(q, num_kv_heads, num_splits, stream):
+    num_seqs, num_q_heads, head_dim = q.shape
+    floats = num_seqs * num_q_heads * num_splits * (head_dim + 2)
+    counters = num_seqs * num_kv_heads * _lib.SPLIT_COUNTER_STRIDE
+    ws = _stream_workspace(q.device, floats, counters, stream)
     return ws.views(num_seqs, num_q_heads, num_splits, head_dim)
 
 
@@ -286,12 +293,15 @@ def paged_decode_attention_into(
     fuse the current token's cache write: the kernel stores it at the slot and
     attends to it from registers.  Mirrors paged_decode.py:972-1264.
 
-    ``ragged=True`` (no counterpart in the reference) tells the library-planned
-    path that the batch's lengths vary widely: each row then gets splits in
+    Without a caller workspace the library plans the launch: large batches are
+    cut into equal shares of tokens whatever the rows' lengths are
+    (``fd_paged_decode_even``), smaller ones give every row the same number of
+    splits.  ``ragged=True`` (no counterpart in the reference) tells the second
+    plan that the batch's lengths vary widely: each row then gets splits in
     proportion to its length, counted on the device from ``seq_lens``
-    (``balance_target`` of the C ABI).  It applies without fused append and
-    without a caller workspace, and only where the batch leaves room in one
-    round of workgroups; elsewhere it changes nothing.
+    (``balance_target`` of the C ABI).  It applies without fused append, and
+    only where the batch leaves room in one round of workgroups; elsewhere it
+    changes nothing.
 
     ``kv_reuse=True`` (no counterpart in the reference) says that rows share
     cache blocks (a common prefix in several rows' tables): K/V are then read
@@ -318,13 +328,20 @@ def paged_decode_attention_into(
     else:
         args, stream = _decode_args(q, k_cache, v_cache, block_tables, seq_lens, out, sm_scale, block_size,
                                     num_warps, kv_layout, num_stages, split_kv_workspace, num_splits, append_k,
-                                    append_v, slot_mapping, ragged, kv_reuse)
+                                    append_v, slot_mapping, ragged, kv_reuse, even=True)
         if key is None:
             key = _launch_key(q, k_cache, v_cache, block_tables, seq_lens, out, split_kv_workspace, append_k,
                               append_v, slot_mapping, (sm_scale, block_size, num_warps, kv_layout, num_stages,
                                                        num_splits, ragged, kv_reuse, stream))
         _LAST_LAUNCH.entry = (key, args)
-    _lib.paged_decode(args, stream)
+    if args.even is None:
+        _lib.paged_decode(args, stream)
+    elif not _lib.paged_decode_even(args, *args.even, stream):
+        # the same shapes and strides at pointers that the even-share kernel does not take
+        args, stream = _decode_args(q, k_cache, v_cache, block_tables, seq_lens, out, sm_scale, block_size,
+                                    num_warps, kv_layout, num_stages, split_kv_workspace, num_splits, append_k,
+                                    append_v, slot_mapping, ragged, kv_reuse)
+        _lib.paged_decode(args, stream)
     return out
 
 
@@ -371,9 +388,11 @@ def _set_pointers(args, q, k_cache, v_cache, block_tables, seq_lens, out, worksp
 
 
 def _decode_args(q, k_cache, v_cache, block_tables, seq_lens, out, sm_scale, block_size, num_warps, kv_layout,
-                 num_stages, split_kv_workspace, num_splits, append_k, append_v, slot_mapping, ragged, kv_reuse):
+                 num_stages, split_kv_workspace, num_splits, append_k, append_v, slot_mapping, ragged, kv_reuse,
+                 even=False):
     """Validation, split plan and workspace of :func:`paged_decode_attention_into`: returns the
-    filled ``PagedDecodeArgs`` and the stream handle, without launching."""
+    filled ``PagedDecodeArgs`` and the stream handle, without launching.  ``even``: the caller
+    launches :func:`_lib.paged_decode_even` where ``args.even`` (its workspace and size) is set."""
     token_axis, dim_axis = _layout_axes(kv_layout)
     if block_size is None:
         if k_cache.dim() != 4:
@@ -441,7 +460,35 @@ def _decode_args(q, k_cache, v_cache, block_tables, seq_lens, out, sm_scale, blo
             raise ValueError("split max and sum workspaces must have identical strides")
     max_seq_len = block_tables.shape[1] * block_size
     stream = _lib.current_stream_handle(q.device)
-    counters = None
+    args = _lib.PagedDecodeArgs()
+    _fill_common(
+        args,
+        q,
+        k_cache,
+        v_cache,
+        _cache_strides(k_cache, token_axis, dim_axis),
+        _cache_strides(v_cache, token_axis, dim_axis),
+        block_tables,
+        seq_lens,
+        out,
+        num_kv_heads,
+        block_size,
+        sm_scale,
+    )
+    args.num_blocks = k_cache.shape[0]
+    args.max_seq_len = max_seq_len
+    args.kv_reuse = 1 if kv_reuse else 0
+    if fuse_kv_append:
+        _fill_append(args, append_k, append_v, slot_mapping)
+    args.even = None
+    if even and not use_split_kv:
+        floats = _lib.paged_decode_even_floats(args)
+        if floats:
+            args.num_splits = 1
+            args.workspace = _stream_workspace(q.device, floats, 0, stream).flat
+            args.even = (args.workspace.data_ptr(), floats)
+            args.caller_workspace = False
+            return args, stream
     balance = 0
     if not use_split_kv:
         if ragged and not fuse_kv_append and use_grouped_gqa:
@@ -464,29 +511,8 @@ def _decode_args(q, k_cache, v_cache, block_tables, seq_lens, out, sm_scale, blo
         split_acc = split_max = split_sum = None
         if num_splits > 1:
             split_acc, split_max, split_sum, _ = _auto_workspace(q, num_kv_heads, num_splits, stream)
-
-    args = _lib.PagedDecodeArgs()
-    _fill_common(
-        args,
-        q,
-        k_cache,
-        v_cache,
-        _cache_strides(k_cache, token_axis, dim_axis),
-        _cache_strides(v_cache, token_axis, dim_axis),
-        block_tables,
-        seq_lens,
-        out,
-        num_kv_heads,
-        block_size,
-        sm_scale,
-    )
-    args.num_blocks = k_cache.shape[0]
-    args.max_seq_len = max_seq_len
     args.balance_target = balance
-    args.kv_reuse = 1 if kv_reuse else 0
-    _fill_workspace(args, split_acc, split_max, split_sum, num_splits, counters)
-    if fuse_kv_append:
-        _fill_append(args, append_k, append_v, slot_mapping)
+    _fill_workspace(args, split_acc, split_max, split_sum, num_splits)
     # the workspace stays alive as long as the arguments that point into it
     # (a later, larger call may replace the stream's own workspace)
     args.workspace = (split_acc, split_max, split_sum)

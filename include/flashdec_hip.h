@@ -304,6 +304,30 @@ int fd_paged_decode_cascade(const fd_paged_decode_args* args, const fd_cascade_a
                             fd_stream_t stream);
 
 /*
+ * fd_paged_decode for batches with enough K/V to fill the GPU, rows of any and
+ * unequal lengths: the batch's tokens are cut into equal shares, one per
+ * workgroup, wherever the row boundaries fall.  No counterpart in the
+ * reference, whose split count is per launch
+ * (flashdec/kernels/paged_decode.py:408-411).
+ *
+ * Same arguments and results as fd_paged_decode with num_splits 1 (the split
+ * workspace fields are not used).  Needs the token-major MFMA path (head_dim 64
+ * or 128, at most 16 query heads per KV head, unit dim strides, 16-byte aligned
+ * rows), strides below 2^31, no fused RoPE, and head_dim 128 with the fused
+ * append; other calls return FD_E_UNSUPPORTED before
+ * anything runs.  workspace: fp32 scratch, 16-byte aligned, at least
+ * fd_paged_decode_even_floats(args) floats (0: the call is not one for this
+ * function), with nothing in it that must be kept between calls; calls that
+ * share one must be ordered on a stream.
+ */
+int fd_paged_decode_even_floats(const fd_paged_decode_args* args);
+/* Whether the library would take fd_paged_decode_even for this call: 1 or 0
+ * (from the shapes and what the block tables can hold; a negative FD_E* code
+ * for a NULL or foreign struct). */
+int fd_paged_decode_even_pays(const fd_paged_decode_args* args);
+int fd_paged_decode_even(const fd_paged_decode_args* args, float* workspace, int64_t floats, fd_stream_t stream);
+
+/*
  * Split count the library would pick for a launch of this shape on the
  * current device (num_splits argument of fd_paged_decode).  max_seq_len is
  * the longest row (or a bound such as max_blocks_per_seq * block_size);

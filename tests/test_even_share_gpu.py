@@ -1,0 +1,139 @@
+"""GPU parity of the even-share decode (``fd_paged_decode_even``): the batch's tokens cut into equal
+shares wherever the row boundaries fall.
+
+The result must equal plain paged decode, so the oracle is the paged-decode oracle, at its tolerance
+(atol 2e-2 / rtol 1e-2).  Cases sit where the shares, segments and merges change form: rows of zero, one,
+31-33 tokens, rows over many shares (the merge's later passes), several rows in one share, batches of more
+than 64 and more than 256 rows (several rows per lane of the length scan), both workgroup widths (256
+(row, KV head) pairs and more take four waves), every block size, head dim and layout the kernel takes.
+The workspace starts as NaN: a merge that reads a slot no workgroup wrote shows.
+"""
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from oracle.attention import paged_decode_attention as oracle_decode
+from tests.helpers import assert_close_to_oracle, make_paged_inputs, np32
+
+pytestmark = pytest.mark.gpu
+
+
+def _even(q, k, v, table, lens, out, append=(None, None, None)):
+    from flashdec_amd import _lib
+    from flashdec_amd.paged_decode import _decode_args
+
+    args, stream = _decode_args(q, k, v, table, lens, out, None, None, 2, "token_major", None, None, 1, *append,
+                                False, False)
+    args.num_splits = 1
+    args.struct_size = ctypes.sizeof(_lib.PagedDecodeArgs)
+    floats = _lib.load_library().fd_paged_decode_even_floats(ctypes.byref(args))
+    assert floats > 0
+    ws = torch.full((floats,), float("nan"), device=q.device)
+    assert _lib.paged_decode_even(args, ws.data_ptr(), floats, stream)
+    torch.cuda.synchronize()
+    return out
+
+
+def _oracle(q, k, v, table, lens):
+    return oracle_decode(np32(q), np32(k), np32(v), table.cpu().numpy(), lens.cpu().numpy())
+
+
+EDGES = [700, 3, 0, 129, 2000, 64, 31, 1, 33, 32, 0, 95]
+MANY = [int(x) for x in np.random.default_rng(5).integers(0, 140, 300)]  # 5 rows per lane of the scan
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("block_size", [8, 16, 32])
+@pytest.mark.parametrize(("hq", "hkv", "d", "lens"), [
+    (16, 2, 128, EDGES),           # 24 pairs: eight waves
+    (16, 1, 128, EDGES),           # 16 heads per KV head
+    (4, 4, 128, EDGES),            # one
+    (14, 2, 64, EDGES),            # 64-dim heads
+    (32, 8, 128, [1]),             # shares past the batch's last
+    (2, 1, 128, [20000, 5]),       # one row over more shares than one merge pass takes
+    (8, 4, 128, MANY),             # 1200 pairs: four waves, several rows a share
+    (8, 1, 64, MANY),
+    (16, 8, 128, [77] * 65),       # uniform rows, one more than the lanes
+])
+def test_even_shares_match_oracle(hq, hkv, d, lens, block_size, dtype):
+    q, k, v, table, sl = make_paged_inputs(lens, hq, hkv, d, block_size, dtype, seed=block_size + hq)
+    out = _even(q, k, v, table, sl, torch.full_like(q, 7.0))
+    assert_close_to_oracle(out, _oracle(q, k, v, table, sl))
+    for b, n in enumerate(lens):
+        if n == 0:
+            assert torch.count_nonzero(out[b]) == 0
+
+
+@pytest.mark.parametrize("block_size", [8, 16, 32])
+def test_even_shares_on_views_wide_tables_and_bad_blocks(block_size):
+    """A vLLM-style cache view, 64-bit indices, tables wider than the rows, lengths past the table, ids outside
+    the pool (masked), and an output with strides of its own."""
+    lens = [40, 0, 333, 5000, 64, 17]
+    q, k, v, table, sl = make_paged_inputs(lens, 16, 2, 128, block_size, seed=3, table_width=5000 // block_size + 9)
+    table[2, 1] = -1
+    table[3, 7] = k.shape[0] + 5
+    sl = sl.long()
+    sl[4] = 10**6  # more than the row's table holds
+    table[4] = table[3]
+    kv = torch.empty((k.shape[0], 2, block_size, 2, 128), device=k.device, dtype=k.dtype)
+    kv[:, 0], kv[:, 1] = k.permute(0, 2, 1, 3), v.permute(0, 2, 1, 3)
+    kview, vview = kv[:, 0].permute(0, 2, 1, 3), kv[:, 1].permute(0, 2, 1, 3)
+    want = _even(q, k, v, table, sl, torch.empty_like(q))
+    wide = torch.zeros((len(lens), 16, 256), device=q.device, dtype=q.dtype)
+    got = _even(q, kview, vview, table.long(), sl, wide[..., ::2])
+    assert torch.equal(got, want)
+    assert torch.count_nonzero(wide[..., 1::2]) == 0
+    from flashdec_amd import paged_decode_attention
+
+    plain = paged_decode_attention(q, k, v, table, sl)  # the row kernel at this size
+    assert_close_to_oracle(want, np32(plain))
+
+
+@pytest.mark.parametrize("block_size", [16, 32])
+@pytest.mark.parametrize("batch", [5, 130])
+def test_even_shares_append_the_current_token(batch, block_size):
+    rng = np.random.default_rng(batch)
+    lens = [int(x) for x in rng.integers(1, 400, batch)]
+    lens[0], lens[1], lens[2] = 1, block_size + 1, 0
+    q, k, v, table, sl = make_paged_inputs(lens, 16, 2, 128, block_size, seed=batch)
+    ak, av = (torch.randn((batch, 2, 128), device="cuda").to(q.dtype) for _ in range(2))
+    pos = (sl.long() - 1).clamp(min=0)
+    slots = table.long().gather(1, (pos // block_size)[:, None])[:, 0] * block_size + pos % block_size
+    slots[3] = -1  # a padding row: nothing written, a zero row
+    slots[2] = 0  # an empty row's slot is not written either
+    k1, v1 = k.clone(), v.clone()
+    out = _even(q, k1, v1, table, sl, torch.empty_like(q), (ak, av, slots))
+    live = [b for b in range(batch) if b not in (2, 3)]
+    ids, off = slots[live] // block_size, slots[live] % block_size
+    k[ids, :, off], v[ids, :, off] = ak[live], av[live]
+    assert torch.equal(k1, k) and torch.equal(v1, v)
+    sl[3] = 0
+    assert_close_to_oracle(out, _oracle(q, k, v, table, sl))
+
+
+def test_large_batches_take_even_shares_and_unaligned_pointers_do_not():
+    """The public call routes by shape; the same shapes at pointers off a 16-byte line keep the general path."""
+    import flashdec_amd as fd
+    from flashdec_amd import _lib
+
+    lens = [900 + 3 * i for i in range(200)]
+    q, k, v, table, sl = make_paged_inputs(lens, 16, 2, 128, 32, seed=1, table_width=1024)
+    _lib.record_launches(True)
+    try:
+        out = fd.decode(q, k, v, table, sl)
+        assert any("even_decode_kernel" in n for n in _lib.last_launch())
+        assert torch.equal(out, fd.decode(q, k, v, table, sl, kv_reuse=True))
+        fd.decode(q, k, v, table[:, :2].contiguous(), sl)  # a small batch
+        assert not any("even" in n for n in _lib.last_launch())
+        assert torch.equal(out, fd.decode(q, k, v, table, sl))
+        flat = torch.empty(q.numel() + 1, device=q.device, dtype=q.dtype)
+        shifted = flat[1:].view(q.shape)
+        shifted.copy_(q)
+        general = fd.decode(shifted, k, v, table, sl)
+        assert not any("even" in n for n in _lib.last_launch())
+    finally:
+        _lib.record_launches(False)
+    assert_close_to_oracle(general, np32(out))
