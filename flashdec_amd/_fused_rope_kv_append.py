@@ -90,14 +90,18 @@ def _validate_structure(q, k, v, k_cache, v_cache, block_ids, block_offsets, pos
     return base
 
 
-def _validate_index_values(block_ids, block_offsets, positions, num_blocks, block_size):
-    """Synchronous device-value checks of the public primitive (:128-145)."""
-    if bool(torch.any(block_ids < 0).item()) or bool(torch.any(block_ids >= num_blocks).item()):
+def _validate_index_values(block_ids, block_offsets, positions, num_blocks, block_size, table_rows=-1):
+    """Synchronous device-value checks of the public primitive (:128-145), one launch for all of them;
+    returns whether a position is past ``table_rows`` (negative: not asked)."""
+    bad_id, bad_offset, bad_position, past_table = _lib.check_append_indices(block_ids, block_offsets, positions,
+                                                                             num_blocks, block_size, table_rows)
+    if bad_id:
         raise ValueError("block_ids must be within [0, num_blocks)")
-    if bool(torch.any(block_offsets < 0).item()) or bool(torch.any(block_offsets >= block_size).item()):
+    if bad_offset:
         raise ValueError("block_offsets must be within [0, block_size)")
-    if bool(torch.any(positions < 0).item()):
+    if bad_position:
         raise ValueError("positions must be non-negative")
+    return past_table
 
 
 def _check_cos_sin_table(table, rotary_dim, device):
@@ -185,10 +189,12 @@ def fused_rope_kv_append(q, k, v, k_cache, v_cache, block_ids, block_offsets, po
     same device bit for bit.  Every position must be below its row count.
     """
     rotary_dim, base = _prepare(q, k, v, k_cache, v_cache, block_ids, block_offsets, positions, rotary_dim, base)
-    _validate_index_values(block_ids, block_offsets, positions, k_cache.shape[0], k_cache.shape[2])
+    # the table's own check comes after the index values', its row count goes along with them
+    rows = cos_sin_table.shape[1] if isinstance(cos_sin_table, torch.Tensor) and cos_sin_table.dim() == 3 else -1
+    past_table = _validate_index_values(block_ids, block_offsets, positions, k_cache.shape[0], k_cache.shape[2], rows)
     if cos_sin_table is not None:
         _check_cos_sin_table(cos_sin_table, rotary_dim, q.device)
-        if bool(torch.any(positions >= cos_sin_table.shape[1]).item()):
+        if past_table:
             raise ValueError("positions must be below the cos_sin_table's rows")
     return _launch(q, k, v, k_cache, v_cache, block_ids, block_offsets, positions, rotary_dim, base,
                    cos_sin_table=cos_sin_table)

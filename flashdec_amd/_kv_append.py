@@ -65,9 +65,11 @@ def _validate_inputs(k_cache, v_cache, block_ids, block_offsets, k, v):
         raise ValueError("K/V caches and values must share one dtype")
     if k_cache.dtype not in _SUPPORTED_DTYPES:
         raise ValueError("CUDA KV append supports float16, bfloat16, and float32")
-    if bool(torch.any(block_ids < 0).item()) or bool(torch.any(block_ids >= k_cache.shape[0]).item()):
+    bad_id, bad_offset, _, _ = _lib.check_append_indices(block_ids, block_offsets, None, k_cache.shape[0],
+                                                         k_cache.shape[2])
+    if bad_id:
         raise ValueError("block_ids must be within [0, num_blocks)")
-    if bool(torch.any(block_offsets < 0).item()) or bool(torch.any(block_offsets >= k_cache.shape[2]).item()):
+    if bad_offset:
         raise ValueError("block_offsets must be within [0, block_size)")
 
 

@@ -126,6 +126,21 @@ class RopeAppendArgs(ctypes.Structure):
     ]
 
 
+class IndexCheckArgs(ctypes.Structure):
+    _fields_ = [
+        ("struct_size", ctypes.c_uint32),
+        ("dtype", _i32 * 3),
+        ("block_ids", _vp),
+        ("block_offsets", _vp),
+        ("positions", _vp),
+        ("count", _i64),
+        ("num_blocks", _i64),
+        ("block_size", _i64),
+        ("table_rows", _i64),
+        ("out", _vp),
+    ]
+
+
 EXPORTED_SYMBOLS = (
     "fd_paged_decode",
     "fd_paged_decode_noalloc",
@@ -138,6 +153,7 @@ EXPORTED_SYMBOLS = (
     "fd_paged_decode_balance_target",
     "fd_fused_rope_kv_append",
     "fd_kv_append",
+    "fd_check_append_indices",
     "fd_last_error",
     "fd_abi_version",
     "fd_record_launches",
@@ -193,6 +209,8 @@ def load_library():
         lib.fd_fused_rope_kv_append.restype = ctypes.c_int
         lib.fd_kv_append.argtypes = [ctypes.POINTER(RopeAppendArgs), _vp]
         lib.fd_kv_append.restype = ctypes.c_int
+        lib.fd_check_append_indices.argtypes = [ctypes.POINTER(IndexCheckArgs), _vp]
+        lib.fd_check_append_indices.restype = ctypes.c_int
         lib.fd_last_error.argtypes = []
         lib.fd_last_error.restype = ctypes.c_char_p
         lib.fd_abi_version.argtypes = []
@@ -340,3 +358,36 @@ def rope_append(args: RopeAppendArgs, stream: int, *, rotate: bool) -> None:
         check(lib.fd_fused_rope_kv_append(ctypes.byref(args), stream), "fd_fused_rope_kv_append")
     else:
         check(lib.fd_kv_append(ctypes.byref(args), stream), "fd_kv_append")
+
+
+# Each thread's result words of check_append_indices (pinned, four int32, and
+# their numpy view): a call fills and reads them before it returns.
+_CHECK_WORDS = threading.local()
+
+
+def check_append_indices(block_ids, block_offsets, positions, num_blocks, block_size, table_rows=-1):
+    """``fd_check_append_indices``: which rules the index values break, after a wait for the stream:
+    (block ids, block offsets, negative positions, positions past ``table_rows``)."""
+    import torch
+
+    words = getattr(_CHECK_WORDS, "words", None)
+    if words is None:
+        pinned = torch.zeros(4, dtype=torch.int32, pin_memory=True)
+        words = _CHECK_WORDS.words = (pinned, pinned.numpy())
+    words[1][:] = 0
+    args = IndexCheckArgs()
+    args.struct_size = ctypes.sizeof(IndexCheckArgs)
+    for k, t in enumerate((block_ids, block_offsets, positions)):
+        if t is not None:
+            args.dtype[k] = index_code(t.dtype)
+    args.block_ids = block_ids.data_ptr()
+    args.block_offsets = block_offsets.data_ptr()
+    args.positions = None if positions is None else positions.data_ptr()
+    args.count = block_ids.numel()
+    args.num_blocks, args.block_size, args.table_rows = num_blocks, block_size, table_rows
+    args.out = words[0].data_ptr()
+    if args.count:
+        stream = current_stream_handle(block_ids.device)
+        with torch.cuda.device(block_ids.device):  # the launch and its wait belong to the tensors' device
+            check(load_library().fd_check_append_indices(ctypes.byref(args), stream), "fd_check_append_indices")
+    return tuple(bool(w) for w in words[1])

@@ -352,6 +352,34 @@ __global__ __launch_bounds__(256) void kv_append_kernel(RopeParams p) {
   }
 }
 
+// Value checks of the index tensors ahead of an append: out[k] becomes 1 where
+// a value breaks rule k (each tensor read once, whatever its integer type;
+// every violation stores the same word, so nothing orders them).  Bound by the
+// launch and the wait for it: one thread per row, a grid-stride loop past 1024
+// workgroups.  Torch reductions with a host round trip each (six, and a seventh
+// for a table) held a 4096-row append to 160 us around its 22 us kernel; with
+// this check the whole call is 43 us.
+struct IndexCheck {
+  const void* data[3];  // block ids, block offsets, positions (may be NULL)
+  int64_t limit[2];     // ids and offsets are within [0, limit)
+  int i64[3];
+  int64_t n;
+  int64_t table_rows;  // >= 0: rule 3, positions below it
+  int32_t* out;
+};
+
+__global__ __launch_bounds__(256) void index_check_kernel(IndexCheck p) {
+  for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < p.n; i += gridDim.x * 256ll) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      if (p.data[k] == nullptr) continue;
+      const int64_t v = p.i64[k] ? static_cast<const int64_t*>(p.data[k])[i] : static_cast<const int32_t*>(p.data[k])[i];
+      if (v < 0 || (k < 2 && v >= p.limit[k])) p.out[k] = 1;
+      if (k == 2 && p.table_rows >= 0 && v >= p.table_rows) p.out[3] = 1;
+    }
+  }
+}
+
 namespace {
 
 int fill_params(const fd_rope_append_args* args, RopeParams& p, bool need_rope, const char* who) {
@@ -460,4 +488,38 @@ extern "C" int fd_kv_append(const fd_rope_append_args* args, fd_stream_t stream_
     case FD_DTYPE_F16: return launch_kv<_Float16>(*args, p, stream);
     default: return launch_kv<float>(*args, p, stream);
   }
+}
+
+extern "C" int fd_check_append_indices(const fd_index_check_args* args, fd_stream_t stream_) {
+  clear_launch_record();
+  static const char* fn = "fd_check_append_indices";
+  if (args == nullptr) return set_error(FD_E_INVALID, "%s: args is NULL", fn);
+  const fd_index_check_args& a = *args;
+  if (a.struct_size != sizeof(fd_index_check_args))
+    return set_error(FD_E_INVALID, "%s: struct_size %u != %zu (ABI mismatch)", fn, a.struct_size,
+                     sizeof(fd_index_check_args));
+  if (a.count < 0 || a.out == nullptr || a.block_ids == nullptr || a.block_offsets == nullptr)
+    return set_error(FD_E_INVALID, "%s: NULL pointer or negative count", fn);
+  if (a.count == 0) return FD_OK;
+  IndexCheck p{};
+  const void* data[3] = {a.block_ids, a.block_offsets, a.positions};
+  for (int k = 0; k < 3; ++k) {
+    p.data[k] = data[k];
+    p.i64[k] = a.dtype[k] == FD_INDEX_I64;
+  }
+  p.limit[0] = a.num_blocks;
+  p.limit[1] = a.block_size;
+  p.n = a.count;
+  p.table_rows = a.table_rows;
+  p.out = a.out;
+  hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
+  const int64_t blocks = (a.count + 255) / 256;
+  if (launch_record_on()) record_launch(reinterpret_cast<const void*>(index_check_kernel), stream);
+  hipLaunchKernelGGL(index_check_kernel, dim3(static_cast<unsigned>(blocks < 1024 ? blocks : 1024)), dim3(256), 0,
+                     stream, p);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return set_error(FD_E_LAUNCH, "%s: launch failed: %s", fn, hipGetErrorString(e));
+  e = hipStreamSynchronize(stream);
+  if (e != hipSuccess) return set_error(FD_E_LAUNCH, "%s: wait failed: %s", fn, hipGetErrorString(e));
+  return FD_OK;
 }

@@ -410,6 +410,31 @@ int fd_fused_rope_kv_append(const fd_rope_append_args* args, fd_stream_t stream)
  */
 int fd_kv_append(const fd_rope_append_args* args, fd_stream_t stream);
 
+/*
+ * Value checks of an append's index tensors (int32 or int64, contiguous, on
+ * the device): one launch and a wait for it on the stream.  out: four int32
+ * words that host and device both reach (pinned host memory), zero before the
+ * call; afterwards out[0] / out[1] / out[2] are 1 where a block id lies outside
+ * [0, num_blocks), an offset outside [0, block_size), a position is negative,
+ * and out[3] where a position is >= table_rows (negative: not checked).
+ * positions may be NULL.  count 0 launches nothing.  No counterpart in the reference, whose
+ * checks are torch reductions (flashdec/_fused_rope_kv_append.py:128-145).
+ */
+typedef struct fd_index_check_args {
+  uint32_t struct_size; /* sizeof(fd_index_check_args): ABI guard */
+  int32_t dtype[3];     /* FD_INDEX_I32 / FD_INDEX_I64: block_ids, block_offsets, positions */
+  const void* block_ids;
+  const void* block_offsets;
+  const void* positions;
+  int64_t count;
+  int64_t num_blocks;
+  int64_t block_size;
+  int64_t table_rows;
+  int32_t* out;
+} fd_index_check_args;
+
+int fd_check_append_indices(const fd_index_check_args* args, fd_stream_t stream);
+
 /* thread-local message for the last failing call on this thread */
 const char* fd_last_error(void);
 
