@@ -227,6 +227,32 @@ def plan_chunk_rows(groups, num_q_heads, num_kv_heads):
     return _lib.CASCADE_MAX_CHUNK_ROWS if rows * groups.max_prefix_len >= _WIDE_CHUNK_MIN_WORK else 16
 
 
+# plan_wide_cascade: KV heads x group rows x prefix tokens from which wide
+# prefix workgroups pay.  Same-box MI355X sweep, us/call, 16- or 32-row chunks
+# (their best) against wide ones at three quarters of the CUs, tails up to 256
+# (Hq/Hkv, sharers x prefix): above the line 16/2 24 x 16384 29.99 vs 25.70,
+# 32/4 24 x 8192 31.30 vs 25.32, 16/1 24 x 16384 26.17 vs 24.53 (6.3 M each),
+# 16/1 64 x 8192 26.01 vs 25.77 (8.4 M, the closest), 32/8 40 x 8192 51.08 vs
+# 32.55, 16/2 64 x 16384 37.08 vs 33.58; below it 16/2 40 x 8192 24.04 vs 23.38,
+# 16/1 40 x 8192 23.54 vs 24.47 (5.2 M), 16/2 24 x 4096 14.62 vs 19.06.  A wide
+# workgroup's time is its fixed part (about 8 us: launch, first loads, merge)
+# and 1.4 us for each 64 tokens.
+_WIDE_TILE_MIN_WORK = 6 << 20
+
+
+def plan_wide_cascade(num_seqs, num_q_heads, num_kv_heads, head_dim, groups, num_cus):
+    """(prefix splits, tail splits) of a launch with wide prefix workgroups
+    (``CASCADE_WIDE_CHUNK_ROWS`` rows each) on three quarters of the CUs, the tails' on the rest, or
+    None where 16- and 32-row chunks are as fast."""
+    rows = groups.max_members * (num_q_heads // num_kv_heads)
+    if head_dim != 128 or groups.num_groups * num_kv_heads * rows * groups.max_prefix_len < _WIDE_TILE_MIN_WORK:
+        return None
+    units = groups.num_groups * num_kv_heads * prefix_chunks(groups, num_q_heads, num_kv_heads,
+                                                             _lib.CASCADE_WIDE_CHUNK_ROWS)
+    tiles = -(-groups.max_prefix_len // 32)
+    return max(1, min(num_cus * 3 // (4 * units), tiles // 4, 1024)), max(1, -(-groups.max_tail_len // 512))
+
+
 def prefix_chunks(groups, num_q_heads, num_kv_heads, chunk_rows=16):
     """Prefix-role chunks per group and KV head: rows (members x query heads per KV head)
     in chunks of ``chunk_rows``, one prefix-role workgroup each."""
@@ -276,7 +302,9 @@ def paged_decode_attention_cascade_into(
     ``[..., >= S + S_p]`` (equal max/sum strides) replaces the library's own,
     e.g. for graph capture.  ``chunk_rows`` (16 or 32; default
     :func:`plan_chunk_rows`) is how many of a group's rows one prefix-role
-    workgroup attends.
+    workgroup attends; with none of ``num_splits``, ``prefix_splits``,
+    ``workspace`` and ``chunk_rows`` given, large groups take wide workgroups
+    (:func:`plan_wide_cascade`).
     """
     key = None
     last = getattr(_LAST_CASCADE, "entry", None)
@@ -326,10 +354,16 @@ def paged_decode_attention_cascade_into(
         raise ValueError("groups.prefix_len must have one entry per group")
     if sm_scale is None:
         sm_scale = 1.0 / math.sqrt(head_dim)
+    wide = None
+    if chunk_rows is None and prefix_splits is None and num_splits is None and workspace is None:
+        wide = plan_wide_cascade(num_seqs, num_q_heads, num_kv_heads, head_dim, groups, _num_cus(q.device))
     if chunk_rows is None:
         chunk_rows = plan_chunk_rows(groups, num_q_heads, num_kv_heads)
     if chunk_rows not in (16, _lib.CASCADE_MAX_CHUNK_ROWS):
         raise ValueError(f"chunk_rows must be 16 or {_lib.CASCADE_MAX_CHUNK_ROWS}")
+    if wide is not None:
+        chunk_rows = _lib.CASCADE_WIDE_CHUNK_ROWS
+        prefix_splits, num_splits = wide
     chunks = prefix_chunks(groups, num_q_heads, num_kv_heads, chunk_rows)
     if prefix_splits is None and num_splits is None:
         prefix_splits, num_splits = plan_cascade_splits(num_seqs, num_q_heads, num_kv_heads, head_dim, groups,

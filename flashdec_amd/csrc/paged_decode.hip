@@ -26,6 +26,7 @@
 #include <mutex>
 
 #include "decode_host.h"
+#include "wide_tile.h"
 
 namespace fd {
 
@@ -1123,6 +1124,69 @@ __global__ __launch_bounds__(64 * waves_for<UNIT>(), 1) void cascade_decode_kern
   }
 }
 
+// The cascade launch with wide prefix workgroups (wide_attend): 128 of a
+// group's (member, head) rows on one read of a prefix split, four row groups of
+// two column blocks by two token groups.  The chunks of one split are
+// consecutive and share an XCD's L2 (xcd_blocks).  Bound by the issue of a
+// batch's phases one after the other (two waves a SIMD, one barrier a batch:
+// 1.4 us per 64 tokens, of which 0.5 are matrix products, 0.6 vector
+// instructions and 0.4 LDS reads).  64 rows on a 16384-token prefix, Hq 16 /
+// Hkv 2: 37.1 -> 33.6 us a call; 40 on 8192, Hq 32 / Hkv 8: 51.1 -> 32.6.
+constexpr int kPrefixRowGroups = 4;
+using PrefixShape = WideShape<128, kPrefixMaxColBlocks, kPrefixRowGroups, 2>;
+static_assert(PrefixShape::kRows == FD_CASCADE_WIDE_CHUNK_ROWS && PrefixShape::kWaves == kMaxWaves);
+
+template <typename T, int BS, bool NT>
+__global__ __launch_bounds__(64 * kMaxWaves, 1) void cascade_wide_kernel(
+    int32_t prefix_wgs, int32_t prefix_splits, int32_t chunks, int32_t hkv, int32_t xcd_blocks,
+    const int32_t* members, int32_t max_members, DecodeParams p, CascadeParams cp) {
+  using TailLds = DecodeLds<waves_for<16>()>;
+  using Lds = WideLds<PrefixShape>;
+  __shared__ alignas(16) uint8_t raw[sizeof(TailLds) > sizeof(Lds) ? sizeof(TailLds) : sizeof(Lds)];
+  if (static_cast<int>(blockIdx.x) >= prefix_wgs) {
+    decode_role<T, BS, false, false, 16, Role::kTail, NT>(p, cp, blockIdx.x - prefix_wgs,
+                                                          *reinterpret_cast<TailLds*>(raw));
+    return;
+  }
+  constexpr int RB = kPrefixMaxColBlocks;
+  const int block = xcd_logical_block(blockIdx.x, xcd_blocks);
+  const int chunk = block % chunks;
+  const int part = block / chunks;
+  const int split = part % prefix_splits;
+  const int gk = part / prefix_splits;
+  const int grp = gk / hkv;
+  // the group's lead, length and this lane's members: one round of loads
+  const int64_t row0 = static_cast<int64_t>(grp) * max_members;
+  const int lead = load_index_uniform(members, row0, 0);
+  const int glen = load_index_uniform(cp.prefix_len, grp, 0);
+  const int rg = (__builtin_amdgcn_readfirstlane(threadIdx.x) >> 6) % kPrefixRowGroups;
+  int32_t m[RB];
+  int col_b[RB], col_h[RB];
+  bool col_ok[RB];
+#pragma unroll
+  for (int cb = 0; cb < RB; ++cb) {
+    const int r = PrefixShape::kRows * chunk + 16 * (RB * rg + cb) + (threadIdx.x & 15);
+    const int mi = r / p.group;
+    col_ok[cb] = mi < max_members;
+    m[cb] = members[row0 + (col_ok[cb] ? mi : 0)];
+    col_h[cb] = r - mi * p.group;
+  }
+  const bool lead_ok = lead >= 0 && lead < p.num_seqs;
+#pragma unroll
+  for (int cb = 0; cb < RB; ++cb) {
+    col_ok[cb] = col_ok[cb] && lead_ok && m[cb] >= 0 && m[cb] < p.num_seqs;
+    col_b[cb] = col_ok[cb] ? m[cb] : 0;
+  }
+  const int plen = lead_ok ? glen : 0;
+  const int64_t cap = p.max_blocks_per_seq * p.block_size;
+  const int64_t eff = plen < 0 ? 0 : (plen < cap ? plen : cap);
+  int t0, t1;
+  split_tiles(prefix_splits, split, eff, 0, t0, t1);
+  const WideWork w{lead_ok ? lead : 0, gk % hkv, 32 * t0, static_cast<int>(min<int64_t>(32 * t1, eff))};
+  wide_attend<T, BS, 128, RB, kPrefixRowGroups, 2, false>(p, w, col_b, col_h, col_ok, p.splits + split,
+                                                          *reinterpret_cast<Lds*>(raw));
+}
+
 // ====================================================== generic path ====
 // One wave per (request, KV head, head group of <= 8 query heads, split).
 // Lane = token within a 64-token tile for QK; lane = dim for PV.
@@ -2034,6 +2098,14 @@ template <typename T, int BS, bool NT>
 void launch_cascade_kernel(const DecodeParams& p, const CascadeParams& cp, int col_blocks, int64_t pairs,
                            hipStream_t stream, void* const* ev) {
   const dim3 grid(static_cast<unsigned>(cp.prefix_blocks + pairs * p.splits));
+  if (col_blocks == FD_CASCADE_WIDE_CHUNK_ROWS / 16) {
+    dispatch(cascade_wide_kernel<T, BS, NT>, grid, dim3(64 * kMaxWaves), stream, ev[0], ev[1],
+             static_cast<int32_t>(cp.prefix_blocks), static_cast<int32_t>(cp.prefix_splits),
+             static_cast<int32_t>(cp.chunks), p.hkv,
+             static_cast<int32_t>(cp.prefix_blocks % 8 == 0 ? cp.prefix_blocks / 8 : 0), cp.members,
+             static_cast<int32_t>(cp.max_members), p, cp);
+    return;
+  }
   if (col_blocks == 2) {
     // long prefixes shared by many rows: 16-token units, two column blocks
     dispatch_cascade(cascade_decode_kernel<T, BS, 16, NT, 2>, grid, dim3(64 * waves_for<16>()), stream, ev, p, cp);
@@ -2484,8 +2556,13 @@ extern "C" int fd_paged_decode_cascade(const fd_paged_decode_args* args, const f
   if (!c.row_prefix_len || (c.num_groups > 0 && (!c.group_members || !c.group_prefix_len)))
     return set_error(FD_E_INVALID, "%s: NULL group pointer", fn);
   if (c.max_prefix_len < 0) return set_error(FD_E_INVALID, "%s: max_prefix_len must be >= 0", fn);
-  if (c.chunk_rows != 0 && c.chunk_rows != 16 && c.chunk_rows != FD_CASCADE_MAX_CHUNK_ROWS)
-    return set_error(FD_E_INVALID, "%s: chunk_rows must be 0, 16 or %d", fn, FD_CASCADE_MAX_CHUNK_ROWS);
+  if (c.chunk_rows != 0 && c.chunk_rows != 16 && c.chunk_rows != FD_CASCADE_MAX_CHUNK_ROWS &&
+      c.chunk_rows != FD_CASCADE_WIDE_CHUNK_ROWS)
+    return set_error(FD_E_INVALID, "%s: chunk_rows must be 0, 16, %d or %d", fn, FD_CASCADE_MAX_CHUNK_ROWS,
+                     FD_CASCADE_WIDE_CHUNK_ROWS);
+  if (c.chunk_rows == FD_CASCADE_WIDE_CHUNK_ROWS && (a.split_acc_stride[3] != 1 || a.num_blocks > INT32_MAX))
+    return set_error(FD_E_UNSUPPORTED, "%s: chunk_rows %d needs unit dim stride of the partials and 32-bit block ids",
+                     fn, FD_CASCADE_WIDE_CHUNK_ROWS);
   const int chunk_rows = c.chunk_rows == 0 ? 16 : c.chunk_rows;
   const int64_t chunks = (static_cast<int64_t>(c.max_members) * p.group + chunk_rows - 1) / chunk_rows;
   const int64_t prefix_blocks = static_cast<int64_t>(c.num_groups) * a.num_kv_heads * chunks * c.prefix_splits;

@@ -281,12 +281,16 @@ int fd_paged_decode_noalloc_prepare(fd_stream_t stream);
  * timing events [0]/[1] bracket the attention launch, [2]/[3] the reducer.
  */
 /* chunk_rows: member x query-head rows of a group that one prefix-role
- * workgroup attends (16 per MFMA column block of its waves), 16 or
- * FD_CASCADE_MAX_CHUNK_ROWS; 0 means 16.  The prefix is read once per
- * chunk; a chunk of 32 rows doubles each wave's work per K/V unit, which pays
- * for long prefixes shared by many rows.  There are ceil(max_members * G /
- * chunk_rows) chunks per (group, KV head). */
+ * workgroup attends (16 per MFMA column block of its waves), 16,
+ * FD_CASCADE_MAX_CHUNK_ROWS or FD_CASCADE_WIDE_CHUNK_ROWS; 0 means 16.  The
+ * prefix is read once per chunk; a chunk of 32 rows doubles each wave's work
+ * per K/V unit, which pays for long prefixes shared by many rows, and a wide
+ * chunk's waves share the tokens through LDS, each with its own rows, which
+ * pays for still more (a caller plans its prefix splits for one workgroup per
+ * CU).  There are ceil(max_members * G / chunk_rows) chunks per (group, KV
+ * head).  Wide chunks need unit dim stride of the split workspace. */
 #define FD_CASCADE_MAX_CHUNK_ROWS 32
+#define FD_CASCADE_WIDE_CHUNK_ROWS 128
 
 typedef struct fd_cascade_args {
   uint32_t struct_size; /* sizeof(fd_cascade_args): ABI guard */
@@ -297,7 +301,7 @@ typedef struct fd_cascade_args {
   const int32_t* group_prefix_len; /* [num_groups], tokens */
   const int32_t* row_prefix_len;   /* [num_seqs], tokens */
   int64_t max_prefix_len;
-  int32_t chunk_rows;              /* 0, 16 or FD_CASCADE_MAX_CHUNK_ROWS (see above) */
+  int32_t chunk_rows;              /* 0, 16, FD_CASCADE_MAX_CHUNK_ROWS or FD_CASCADE_WIDE_CHUNK_ROWS */
 } fd_cascade_args;
 
 int fd_paged_decode_cascade(const fd_paged_decode_args* args, const fd_cascade_args* cascade,
