@@ -236,21 +236,29 @@ def plan_chunk_rows(groups, num_q_heads, num_kv_heads):
 # 32.55, 16/2 64 x 16384 37.08 vs 33.58; below it 16/2 40 x 8192 24.04 vs 23.38,
 # 16/1 40 x 8192 23.54 vs 24.47 (5.2 M), 16/2 24 x 4096 14.62 vs 19.06.  A wide
 # workgroup's time is its fixed part (about 8 us: launch, first loads, merge)
-# and 1.4 us for each 64 tokens.
+# and 1.4 us for each 64 tokens.  One tail split always measured best beside
+# them, and a tail-role workgroup then outlasts the prefix role's past 512
+# tokens: 32/4 24 x 8192 34.33 vs 25.44 with tails to 512, 32.98 vs 27.20 to
+# 1024; 16/2 64 x 8192 29.29 vs 25.95, 31.85 vs 31.79; 16/2 64 x 16384 39.14 vs
+# 34.11, 40.55 vs 34.04.  Longer tails keep the 32-row chunks, which
+# tests/test_routing_gpu.py holds 64 x 16384 with tails to 700 to.
 _WIDE_TILE_MIN_WORK = 6 << 20
+_WIDE_TILE_MAX_TAIL = 512
 
 
 def plan_wide_cascade(num_seqs, num_q_heads, num_kv_heads, head_dim, groups, num_cus):
     """(prefix splits, tail splits) of a launch with wide prefix workgroups
     (``CASCADE_WIDE_CHUNK_ROWS`` rows each) on three quarters of the CUs, the tails' on the rest, or
-    None where 16- and 32-row chunks are as fast."""
+    None for 16- and 32-row chunks."""
+    if groups.max_tail_len > _WIDE_TILE_MAX_TAIL:
+        return None
     rows = groups.max_members * (num_q_heads // num_kv_heads)
     if head_dim != 128 or groups.num_groups * num_kv_heads * rows * groups.max_prefix_len < _WIDE_TILE_MIN_WORK:
         return None
     units = groups.num_groups * num_kv_heads * prefix_chunks(groups, num_q_heads, num_kv_heads,
                                                              _lib.CASCADE_WIDE_CHUNK_ROWS)
     tiles = -(-groups.max_prefix_len // 32)
-    return max(1, min(num_cus * 3 // (4 * units), tiles // 4, 1024)), max(1, -(-groups.max_tail_len // 512))
+    return max(1, min(num_cus * 3 // (4 * units), tiles // 4, 1024)), 1
 
 
 def prefix_chunks(groups, num_q_heads, num_kv_heads, chunk_rows=16):

@@ -44,15 +44,16 @@ def test_wide_chunks_match_oracle(heads, sharers, blocks, block_size, dtype, pla
 
 
 def test_plan_and_explicit_settings():
-    def groups(members, prefix):
+    def groups(members, prefix, tail=512):
         return cascade.CascadeGroups(members=torch.zeros((1, members), dtype=torch.int32),
                                      prefix_len=torch.zeros(1, dtype=torch.int32),
                                      row_prefix_len=torch.zeros(members, dtype=torch.int32), max_prefix_len=prefix,
-                                     max_tail_len=600, total_tail_len=1)
+                                     max_tail_len=tail, total_tail_len=1)
 
-    assert cascade.plan_wide_cascade(64, 16, 2, 128, groups(64, 16384), 256) == (24, 2)  # 8 units, 192 workgroups
-    assert cascade.plan_wide_cascade(24, 32, 4, 128, groups(24, 8192), 256) == (24, 2)  # exactly 6 * 2^20
+    assert cascade.plan_wide_cascade(64, 16, 2, 128, groups(64, 16384), 256) == (24, 1)  # 8 units, 192 workgroups
+    assert cascade.plan_wide_cascade(24, 32, 4, 128, groups(24, 8192), 256) == (24, 1)  # exactly 6 * 2^20
     assert cascade.plan_wide_cascade(23, 32, 4, 128, groups(23, 8192), 256) is None
+    assert cascade.plan_wide_cascade(64, 16, 2, 128, groups(64, 16384, 513), 256) is None
     # explicit settings keep what they took and refused
     q, k, v, table, lens, _ = make_prefix_inputs([(4, [5, 6])], [], 16, 2, 16, torch.bfloat16)
     g = cascade.build_cascade_groups(table, lens, 16, 16, 2)
