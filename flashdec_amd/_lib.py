@@ -286,10 +286,15 @@ def current_stream_handle(device) -> int:
     return raw(torch.cuda.current_device() if device.index is None else device.index)
 
 
+_PAGED_DECODE_BYTES = ctypes.sizeof(PagedDecodeArgs)
+
+
 def paged_decode(args: PagedDecodeArgs, stream: int) -> None:
-    lib = load_library()
-    args.struct_size = ctypes.sizeof(PagedDecodeArgs)
-    check(lib.fd_paged_decode(ctypes.byref(args), stream), "fd_paged_decode")
+    lib = _lib or load_library()
+    args.struct_size = _PAGED_DECODE_BYTES
+    rc = lib.fd_paged_decode(ctypes.byref(args), stream)
+    if rc:
+        check(rc, "fd_paged_decode")
 
 
 def paged_decode_noalloc_prepare(stream: int) -> None:

@@ -252,6 +252,8 @@ def plan_wide_cascade(num_seqs, num_q_heads, num_kv_heads, head_dim, groups, num
     None for 16- and 32-row chunks."""
     if groups.max_tail_len > _WIDE_TILE_MAX_TAIL:
         return None
+    if num_seqs * num_q_heads * groups.max_prefix_len < _WIDE_TILE_MIN_WORK:
+        return None  # fewer rows than that in all: no look at the index tensors' shapes
     rows = groups.max_members * (num_q_heads // num_kv_heads)
     if head_dim != 128 or groups.num_groups * num_kv_heads * rows * groups.max_prefix_len < _WIDE_TILE_MIN_WORK:
         return None

@@ -322,7 +322,7 @@ def paged_decode_attention_into(
     if key is not None and last[0] == key:
         # the previous call's shapes, strides, dtypes, devices and settings:
         # its validation and plan stand; only the data pointers change
-        args = last[1]
+        _, args, even = last
         _set_pointers(args, q, k_cache, v_cache, block_tables, seq_lens, out, split_kv_workspace, append_k,
                       append_v, slot_mapping)
     else:
@@ -333,10 +333,11 @@ def paged_decode_attention_into(
             key = _launch_key(q, k_cache, v_cache, block_tables, seq_lens, out, split_kv_workspace, append_k,
                               append_v, slot_mapping, (sm_scale, block_size, num_warps, kv_layout, num_stages,
                                                        num_splits, ragged, kv_reuse, stream))
-        _LAST_LAUNCH.entry = (key, args)
-    if args.even is None:
+        even = args.even
+        _LAST_LAUNCH.entry = (key, args, even)
+    if even is None:
         _lib.paged_decode(args, stream)
-    elif not _lib.paged_decode_even(args, *args.even, stream):
+    elif not _lib.paged_decode_even(args, *even, stream):
         # the same shapes and strides at pointers that the even-share kernel does not take
         args, stream = _decode_args(q, k_cache, v_cache, block_tables, seq_lens, out, sm_scale, block_size,
                                     num_warps, kv_layout, num_stages, split_kv_workspace, num_splits, append_k,
@@ -345,7 +346,7 @@ def paged_decode_attention_into(
     return out
 
 
-# The last launch of each thread: (metadata key, PagedDecodeArgs).
+# The last launch of each thread: (metadata key, PagedDecodeArgs, its even).
 _LAST_LAUNCH = threading.local()
 
 
@@ -481,7 +482,8 @@ def _decode_args(q, k_cache, v_cache, block_tables, seq_lens, out, sm_scale, blo
     if fuse_kv_append:
         _fill_append(args, append_k, append_v, slot_mapping)
     args.even = None
-    if even and not use_split_kv:
+    # (a batch of fewer than 4096 tiles is below every line of the library's rule: no call to ask it)
+    if even and not use_split_kv and num_seqs * num_kv_heads * -(-max_seq_len // 32) * head_dim >= 4096 * 128:
         floats = _lib.paged_decode_even_floats(args)
         if floats:
             args.num_splits = 1
