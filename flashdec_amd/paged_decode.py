@@ -191,30 +191,42 @@ class _SplitWorkspace:
 _WORKSPACES = {}
 
 
-def _stream_workspace(device, floats, counters, stream):
-    """This stream's workspace, grown to the sizes asked for; a private one inside a graph capture
-    that it is too small for."""
-    key = (device.index, stream)
-    ws = _WORKSPACES.get(key)
-    if ws is None or ws.flat.numel() < floats or ws.counters.numel() < counters:
-        if torch.cuda.is_current_stream_capturing():
-            return _SplitWorkspace(device, floats, counters)
-        grow = 1 if ws is None else 2
-        ws = _SplitWorkspace(
-            device,
-            max(floats, grow * (ws.flat.numel() if ws else 0)),
-            max(counters, grow * (ws.counters.numel() if ws else 0)),
-        )
-        _WORKSPACES[key] = ws
-    return ws
-
-
 def _auto_workspace(q, num_kv_heads, num_splits, stream):
     num_seqs, num_q_heads, head_dim = q.shape
     floats = num_seqs * num_q_heads * num_splits * (head_dim + 2)
     counters = num_seqs * num_kv_heads * _lib.SPLIT_COUNTER_STRIDE
-    ws = _stream_workspace(q.device, floats, counters, stream)
+    key = (q.device.index, stream)
+    ws = _WORKSPACES.get(key)
+    if ws is None or ws.flat.numel() < floats or ws.counters.numel() < counters:
+        if torch.cuda.is_current_stream_capturing():
+            return _SplitWorkspace(q.device, floats, counters).views(num_seqs, num_q_heads, num_splits, head_dim)
+        grow = 1 if ws is None else 2
+        ws = _SplitWorkspace(
+            q.device,
+            max(floats, grow * (ws.flat.numel() if ws else 0)),
+            max(counters, grow * (ws.counters.numel() if ws else 0)),
+        )
+        _WORKSPACES[key] = ws
     return ws.views(num_seqs, num_q_heads, num_splits, head_dim)
+
+
+# Each thread's even-share workspaces, one per (device, stream), 8.6 MB at most
+# each: two threads' launches on one stream may fall between each other's
+# attention and reducer, so they share none.
+_EVEN_WORKSPACES = threading.local()
+
+
+def _even_workspace(device, floats, stream):
+    """fp32 scratch of one even-share call.  Looked up per call, and inside a graph capture allocated
+    for that call alone: it then belongs to the graph's memory, so that no later call writes it between
+    replays and none outlives it."""
+    if torch.cuda.is_current_stream_capturing():
+        return torch.empty(floats, device=device, dtype=torch.float32)
+    held = _EVEN_WORKSPACES.__dict__
+    ws = held.get((device.index, stream))
+    if ws is None or ws.numel() < floats:
+        ws = held[(device.index, stream)] = torch.empty(floats, device=device, dtype=torch.float32)
+    return ws
 
 
 def paged_decode_attention(
@@ -335,9 +347,11 @@ def paged_decode_attention_into(
                                                        num_splits, ragged, kv_reuse, stream))
         even = args.even
         _LAST_LAUNCH.entry = (key, args, even)
-    if even is None:
+    if not even:
         _lib.paged_decode(args, stream)
-    elif not _lib.paged_decode_even(args, *even, stream):
+        return out
+    ws = _even_workspace(q.device, even, stream)
+    if not _lib.paged_decode_even(args, ws.data_ptr(), even, stream):
         # the same shapes and strides at pointers that the even-share kernel does not take
         args, stream = _decode_args(q, k_cache, v_cache, block_tables, seq_lens, out, sm_scale, block_size,
                                     num_warps, kv_layout, num_stages, split_kv_workspace, num_splits, append_k,
@@ -346,7 +360,8 @@ def paged_decode_attention_into(
     return out
 
 
-# The last launch of each thread: (metadata key, PagedDecodeArgs, its even).
+# The last launch of each thread: (metadata key, PagedDecodeArgs, its even-share
+# workspace's floats).
 _LAST_LAUNCH = threading.local()
 
 
@@ -393,7 +408,7 @@ def _decode_args(q, k_cache, v_cache, block_tables, seq_lens, out, sm_scale, blo
                  even=False):
     """Validation, split plan and workspace of :func:`paged_decode_attention_into`: returns the
     filled ``PagedDecodeArgs`` and the stream handle, without launching.  ``even``: the caller
-    launches :func:`_lib.paged_decode_even` where ``args.even`` (its workspace and size) is set."""
+    launches :func:`_lib.paged_decode_even` where ``args.even`` (the floats of its workspace) is not 0."""
     token_axis, dim_axis = _layout_axes(kv_layout)
     if block_size is None:
         if k_cache.dim() != 4:
@@ -481,14 +496,13 @@ def _decode_args(q, k_cache, v_cache, block_tables, seq_lens, out, sm_scale, blo
     args.kv_reuse = 1 if kv_reuse else 0
     if fuse_kv_append:
         _fill_append(args, append_k, append_v, slot_mapping)
-    args.even = None
+    args.even = 0
     # (a batch of fewer than 4096 tiles is below every line of the library's rule: no call to ask it)
     if even and not use_split_kv and num_seqs * num_kv_heads * -(-max_seq_len // 32) * head_dim >= 4096 * 128:
         floats = _lib.paged_decode_even_floats(args)
         if floats:
             args.num_splits = 1
-            args.workspace = _stream_workspace(q.device, floats, 0, stream).flat
-            args.even = (args.workspace.data_ptr(), floats)
+            args.even = floats
             args.caller_workspace = False
             return args, stream
     balance = 0

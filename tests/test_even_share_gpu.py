@@ -137,3 +137,49 @@ def test_large_batches_take_even_shares_and_unaligned_pointers_do_not():
     finally:
         _lib.record_launches(False)
     assert_close_to_oracle(general, np32(out))
+
+
+def test_even_share_workspaces_are_a_graphs_own_and_a_threads_own():
+    """A captured call's partials stay in the graph's memory whatever the stream ran before, and threads on
+    one stream have a workspace each."""
+    import threading
+
+    import flashdec_amd as fd
+    from flashdec_amd import paged_decode as pd
+
+    q, k, v, table, sl = make_paged_inputs([900 + 3 * i for i in range(200)], 16, 2, 128, 32, seed=2,
+                                           table_width=1024)
+    held = pd._EVEN_WORKSPACES.__dict__
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        want = fd.decode(q, k, v, table, sl)
+        ws = held[(q.device.index, side.cuda_stream)]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = fd.decode(q, k, v, table, sl)
+    assert held[(q.device.index, side.cuda_stream)] is ws
+    for _ in range(3):
+        ws.fill_(7.0)
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        assert bool((ws == 7.0).all())
+        with torch.cuda.stream(side):  # the same call again, eager: the stream's own workspace, not the graph's
+            assert torch.equal(fd.decode(q, k, v, table, sl), want)
+        torch.cuda.synchronize()
+        assert not bool((ws == 7.0).all())
+    seen = []
+
+    def other():
+        with torch.cuda.stream(side):
+            seen.append(fd.decode(q, k, v, table, sl))
+        seen.append(pd._EVEN_WORKSPACES.__dict__[(q.device.index, side.cuda_stream)].data_ptr())
+        torch.cuda.synchronize()
+
+    t = threading.Thread(target=other)
+    t.start()
+    t.join()
+    assert torch.equal(seen[0], want) and seen[1] != ws.data_ptr()
