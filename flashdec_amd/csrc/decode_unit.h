@@ -516,17 +516,22 @@ __device__ __forceinline__ float tree_sum16(const float (&x)[16]) {
 // overflow in fp32, the same relative rounding in the cache dtype), and the
 // accumulator's multiply runs only on such moves instead of on most units.
 // acc and l are always taken against the same st.m, so the partial they
-// stand for is the same up to rounding.
+// stand for is the same up to rounding.  LAZY false moves the maximum to every
+// new one, so that a peak's probability is 1 and the cache dtype holds it
+// exactly (even_decode.hip, whose waves take more units of a row: relative
+// error against 64 bits 0.0022 lazy, 0.0018 not, for 193 rows of 256 .. 511
+// tokens in bf16, where the row kernel has 0.0019; 54.6 us either way, the
+// rescales hide behind the loads).
 constexpr float kRescaleSlack = 8.f;
 
-template <int VR, int D>
+template <int VR, int D, bool LAZY = true>
 __device__ __forceinline__ void softmax_step(const float (&sc)[VR], float (&pr)[VR], WaveState<D>& st) {
   float mx = sc[0];
 #pragma unroll
   for (int i = 1; i < VR; ++i) mx = fmaxf(mx, sc[i]);
   mx = column_max(mx);
   // st.m == -inf: -inf + slack is -inf, so the first live unit moves it
-  const bool move = mx > st.m + kRescaleSlack;
+  const bool move = mx > (LAZY ? st.m + kRescaleSlack : st.m);
   const float m_ref = move ? mx : st.m;
   const float m_use = m_ref == -INFINITY ? 0.f : m_ref;
   float psum = 0.f;
@@ -555,7 +560,7 @@ __device__ __forceinline__ void softmax_step(const float (&sc)[VR], float (&pr)[
 // reference's grouped kernels do (flashdec/kernels/paged_decode.py:308-310);
 // the denominator sums them in fp32.  Masking is skipped for units whose
 // tokens are all live (wave-uniform test).
-template <typename T, bool FUSE, int UNIT, int D, int NCB, bool TL = false>
+template <typename T, bool FUSE, int UNIT, int D, int NCB, bool TL = false, bool LAZY = true>
 __device__ __forceinline__ void process_unit(UnitRegs<UNIT, D>& t, const u32x4 (&qf)[NCB][D / 32],
                                              float scale_log2, int tok0, int first, int last, int app,
                                              const AppendRegs<D>& ar, int c, int g, WaveState<D> (&st)[NCB]) {
@@ -619,7 +624,7 @@ __device__ __forceinline__ void process_unit(UnitRegs<UNIT, D>& t, const u32x4 (
 #pragma unroll
   for (int cb = 0; cb < NCB; ++cb) {
     float pr[VR];
-    softmax_step<VR, D>(sc[cb], pr, st[cb]);
+    softmax_step<VR, D, LAZY>(sc[cb], pr, st[cb]);
 #pragma unroll
     for (int j = 0; j < VR / 2; ++j) ph[cb][j] = pack2<T>(pr[2 * j], pr[2 * j + 1]);
   }

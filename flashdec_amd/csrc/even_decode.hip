@@ -551,8 +551,8 @@ __global__ __launch_bounds__(64 * W, kEvenWavesPerCU / W) void even_decode_kerne
         even_store_append<T, BS, D>(a, cur.kvh, slot, c, g, ar);
       }
     }
-    process_unit<T, FUSE, UNIT, D, 1>(now, qf, a.scale_log2, UNIT * cur.unit, 0, min(cur.len, 32 * cur.t_end) - 1, app,
-                                        ar, c, g, st);
+    process_unit<T, FUSE, UNIT, D, 1, false, false>(now, qf, a.scale_log2, UNIT * cur.unit, 0,
+                                                    min(cur.len, 32 * cur.t_end) - 1, app, ar, c, g, st);
     if (last) {
       if (more) load_q(nxt, qf);  // in flight during the merge
       flush(cur);
