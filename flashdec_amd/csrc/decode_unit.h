@@ -518,10 +518,11 @@ __device__ __forceinline__ float tree_sum16(const float (&x)[16]) {
 // acc and l are always taken against the same st.m, so the partial they
 // stand for is the same up to rounding.  LAZY false moves the maximum to every
 // new one, so that a peak's probability is 1 and the cache dtype holds it
-// exactly (even_decode.hip, whose waves take more units of a row: relative
-// error against 64 bits 0.0022 lazy, 0.0018 not, for 193 rows of 256 .. 511
-// tokens in bf16, where the row kernel has 0.0019; 54.6 us either way, the
-// rescales hide behind the loads).
+// exactly: even_decode.hip and wide_tile.h, whose waves take more units of a
+// row (relative error against 64 bits, bf16, lazy / not / row kernels: 193 rows
+// of 256 .. 511 tokens 0.0022 / 0.0018 / 0.0019, 54.6 us either way, the rescales
+// hide behind the loads; 64 rows on a 16384-token prefix 0.0022 / 0.0018 /
+// 0.0021, 30.5 / 32.5 / 34.2 us).
 constexpr float kRescaleSlack = 8.f;
 
 template <int VR, int D, bool LAZY = true>

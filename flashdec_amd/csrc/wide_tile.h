@@ -207,7 +207,7 @@ __device__ __forceinline__ void wide_compute(const u32x4 (&qf)[RB][D / 32], floa
 #pragma unroll
   for (int cb = 0; cb < RB; ++cb) {
     float pr[8];
-    softmax_step<8, D>(sc[cb], pr, st[cb]);
+    softmax_step<8, D, false>(sc[cb], pr, st[cb]);
 #pragma unroll
     for (int j = 0; j < 4; ++j) ph[cb][j] = pack2<T>(pr[2 * j], pr[2 * j + 1]);
   }

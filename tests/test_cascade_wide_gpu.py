@@ -43,6 +43,32 @@ def test_wide_chunks_match_oracle(heads, sharers, blocks, block_size, dtype, pla
     assert torch.count_nonzero(out[sharers + 2]) == 0  # the zero-length row
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize(("heads", "sharers", "blocks"), [((16, 2), 64, 256), ((32, 8), 40, 128)])
+def test_wide_chunks_are_no_further_from_64_bits_than_32_row_chunks(heads, sharers, blocks, dtype, monkeypatch):
+    """Peaked scores (queries of twice unit size): a wave of a wide workgroup takes more tokens of a row than one
+    of a 32-row chunk does, and a peak's probability rounds to the cache type all the same."""
+    hq, hkv = heads
+    q, k, v, table, lens, _ = make_prefix_inputs([(blocks, [(37 * i) % 200 + 1 for i in range(sharers)])], [], hq, hkv,
+                                                 32, dtype)
+    q = q * 2
+    g = cascade.build_cascade_groups(table, lens, 32, hq, hkv)
+    narrow = cascade.paged_decode_attention_cascade(q, k, v, table, lens, groups=g, chunk_rows=32)
+    monkeypatch.setattr(cascade, "plan_wide_cascade", lambda *a: (24, 1))
+    monkeypatch.setattr(cascade, "_LAST_CASCADE", type(cascade._LAST_CASCADE)())
+    wide = cascade.paged_decode_attention_cascade(q, k, v, table, lens, groups=g)
+    exact = torch.empty(q.shape, device=q.device, dtype=torch.float64)
+    for b, n in enumerate(lens.tolist()):
+        ids = table[b, : -(-n // 32)].long()
+        for h in range(hkv):
+            kh, vh = (t[ids, h].reshape(-1, 128)[:n].double() for t in (k, v))
+            qh = q[b, h * (hq // hkv) : (h + 1) * (hq // hkv)].double()
+            p = torch.softmax((kh @ qh.t().contiguous()).t() / math.sqrt(128), dim=-1)
+            exact[b, h * (hq // hkv) : (h + 1) * (hq // hkv)] = p.contiguous() @ vh
+    off = [float((t.double() - exact).norm() / exact.norm()) for t in (wide, narrow)]
+    assert off[0] <= off[1], off
+
+
 def test_plan_and_explicit_settings():
     def groups(members, prefix, tail=512):
         return cascade.CascadeGroups(members=torch.zeros((1, members), dtype=torch.int32),
