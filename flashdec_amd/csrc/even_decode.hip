@@ -284,11 +284,7 @@ __global__ __launch_bounds__(64 * W, kEvenWavesPerCU / W) void even_decode_kerne
     const int tiles = even_tiles(cu.len);
     const bool whole = cu.t_begin == 0 && cu.t_end == tiles;
     const int slot = 2 * share + (cu.t_begin == 0 ? 1 : 0);
-    if (cu.left == 0 && threadIdx.x == 0) {
-      const bool starts = cu.t_begin == 0 && !whole;
-      const int parts = (share_end - cu.t_end + tiles - 1) / per - share + 1;
-      w.cuts[share] = EvenCut{cu.b, cu.kvh, starts ? parts : 0, 0};
-    }
+    if (cu.left == 0 && threadIdx.x == 0) w.cuts[share] = even_cut(cu, tiles, whole, share, share_end, per);
     const float lt = column_sum(st[0].l);
     if (g == 0) {
       s_m[set][wave][c] = st[0].m;
@@ -380,11 +376,11 @@ constexpr int kEvenParts = 16;
 
 template <typename T, int D, int EARLY>
 __global__ __launch_bounds__(256) void even_reduce_kernel(const EvenCut* cuts, const float* acc, const float* stats,
-                                                          int32_t heads, EvenOut w) {
+                                                          int32_t heads, int32_t shares, int32_t num_seqs, int32_t hkv,
+                                                          EvenOut w) {
   constexpr int N = 4;  // dims per thread
   constexpr int kDimThreads = D / N;
   const int share = blockIdx.x;
-  const EvenCut cut = cuts[share];
   struct Part {
     f32x4 x;
     float2 ml;
@@ -402,24 +398,27 @@ __global__ __launch_bounds__(256) void even_reduce_kernel(const EvenCut* cuts, c
     Part early[EARLY];
 #pragma unroll
     for (int j = 0; j < EARLY; ++j) early[j] = part(j);
-    if (cut.parts == 0) return;
+    asm volatile("" ::: "memory");  // the cut's load and its tests stay behind those loads
+    const EvenCut cut = cuts[share];
+    const int parts = even_cut_parts(cut, share, shares, num_seqs, hkv);
+    if (parts <= 0) return;
     float M = -INFINITY, L = 0.f;
 #pragma unroll
-    for (int j = 0; j < EARLY; ++j) M = j < cut.parts ? fmaxf(M, early[j].ml.x) : M;
+    for (int j = 0; j < EARLY; ++j) M = j < parts ? fmaxf(M, early[j].ml.x) : M;
     float mu = M == -INFINITY ? 0.f : M;
     float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < EARLY; ++j) {
-      if (j >= cut.parts) continue;
+      if (j >= parts) continue;
       const float wt = exp2_fast(early[j].ml.x - mu);
       L += wt * early[j].ml.y;
 #pragma unroll
       for (int k = 0; k < N; ++k) o[k] += wt * early[j].x[k];
     }
-    for (int j0 = EARLY; j0 < cut.parts; j0 += kEvenParts) {
+    for (int j0 = EARLY; j0 < parts; j0 += kEvenParts) {
       Part p[kEvenParts];
 #pragma unroll
-      for (int j = 0; j < kEvenParts; ++j) p[j] = part(min(j0 + j, cut.parts - 1));
+      for (int j = 0; j < kEvenParts; ++j) p[j] = part(min(j0 + j, parts - 1));
       float nm = M;
 #pragma unroll
       for (int j = 0; j < kEvenParts; ++j) nm = fmaxf(nm, p[j].ml.x);  // past the end: a part again, weight 0
@@ -430,7 +429,7 @@ __global__ __launch_bounds__(256) void even_reduce_kernel(const EvenCut* cuts, c
       for (int k = 0; k < N; ++k) o[k] *= sc;
 #pragma unroll
       for (int j = 0; j < kEvenParts; ++j) {
-        const float wt = j0 + j < cut.parts ? exp2_fast(p[j].ml.x - mu) : 0.f;
+        const float wt = j0 + j < parts ? exp2_fast(p[j].ml.x - mu) : 0.f;
         L += wt * p[j].ml.y;
 #pragma unroll
         for (int k = 0; k < N; ++k) o[k] += wt * p[j].x[k];
@@ -526,7 +525,7 @@ int launch_even(const fd_paged_decode_args& a, const EvenArgs& e, const EvenOut&
     const unsigned per_share = static_cast<unsigned>((w.heads * a.head_dim / 4 + 255) / 256);
     dispatch(kernel, dim3(static_cast<unsigned>(e.shares), per_share), dim3(256), stream, a.timing_events[2],
              a.timing_events[3], static_cast<const EvenCut*>(w.cuts), static_cast<const float*>(w.acc),
-             static_cast<const float*>(w.stats), w.heads, w);
+             static_cast<const float*>(w.stats), w.heads, e.shares, e.num_seqs, e.hkv, w);
   };
   if (waves == 8)
     a.head_dim == 64 ? reduce(even_reduce_kernel<T, 64, 4>) : reduce(even_reduce_kernel<T, 128, 4>);

@@ -1,6 +1,12 @@
 // The even-share kernel's line of tiles: which part of it a workgroup takes and
 // how its waves walk that part.  Integer logic over the rows' lengths only; the
-// includer brings the index loads and the lane operations.
+// includer brings the index loads and the lane operations (tests/native runs it
+// on the host).
+//
+// Each wave reads the lengths for itself, some of them twice, so a caller that
+// changes them under the launch (the next step's update on another stream) may
+// show it different ones.  Its rows are then wrong, as any kernel's would be, but
+// every walk ends, and every row, slot and part stays in range.
 #pragma once
 
 namespace fd {
@@ -175,7 +181,8 @@ __device__ __forceinline__ EvenCursor even_first(const EvenArgs& a, int block, i
   int base = __builtin_amdgcn_readlane(incl - mine, l);
   int b = l * n;
   int row_len = __builtin_amdgcn_readlane(len, l);
-  for (int i = 0; n > 1; i += 64) {  // the row among the lane's own
+  // the row among the lane's own (if none is it, a length changed since the scan)
+  for (int i = 0; n > 1 && i < n; i += 64) {
     const int r = l * n + i + lane;
     const bool in = i + lane < n && r < a.num_seqs;
     const int rl = even_row_len<FUSE, false>(a, in ? r : 0);
@@ -200,6 +207,25 @@ __device__ __forceinline__ EvenCursor even_first(const EvenArgs& a, int block, i
   c.t_end = min(tiles, c.t_begin + c.left);
   c.left -= c.t_end - c.t_begin;
   return c;
+}
+
+// The cut of a share whose last segment is cu's.
+__device__ __forceinline__ EvenCut even_cut(const EvenCursor& cu, int tiles, bool whole, int share, int share_end,
+                                            int per) {
+  const bool starts = cu.t_begin == 0 && !whole;
+  const int parts = (share_end - cu.t_end + tiles - 1) / per - share + 1;
+  return EvenCut{cu.b, cu.kvh, starts ? parts : 0, 0};
+}
+
+// Parts that a share's merge takes, 0 or less for no merge.  The cut may be one
+// that no workgroup of this launch wrote (lengths that changed: a walk that ended
+// early, another share than the workgroup's id stands for): whatever it holds,
+// the parts end with the last share's and the row is one of the batch's.
+__device__ __forceinline__ int even_cut_parts(const EvenCut& cut, int share, int shares, int num_seqs, int hkv) {
+  // (one load of the cut and no branch before the parts are known)
+  const bool row = (static_cast<uint32_t>(cut.b) < static_cast<uint32_t>(num_seqs)) &
+                   (static_cast<uint32_t>(cut.kvh) < static_cast<uint32_t>(hkv));
+  return min(cut.parts, shares - share) & -static_cast<int>(row);
 }
 
 }  // namespace fd
