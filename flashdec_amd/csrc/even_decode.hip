@@ -230,9 +230,9 @@ __global__ __launch_bounds__(64 * W, kEvenWavesPerCU / W) void even_decode_kerne
   }
   const UnitPages guessed = even_pages<BS, UNIT>(a, guess);
   if constexpr (FUSE) raw_len = raw_slot < 0 ? 0 : raw_len;
-  int share, per, share_end;
+  int share, per, share_end, pad;
   EvenCursor cur =
-      even_first<FUSE>(a, blockIdx.x, lane, min(max(raw_len, 0), a.cap), share, per, share_end);
+      even_first<FUSE>(a, blockIdx.x, lane, min(max(raw_len, 0), a.cap), share, per, share_end, pad);
   if (!cur.valid) {  // every wave of the workgroup
     if (threadIdx.x == 0) out_args().cuts[share].parts = 0;
     return;
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(64 * W, kEvenWavesPerCU / W) void even_decode_kerne
   if (cur.b != guess.b || cur.unit != guess.unit || !guess.valid) pages = even_pages<BS, UNIT>(a, cur);
   load_q(cur, qf);
   even_load<T, BS, UNIT, D, NT>(a, cur, pages, c, g, ra);
-  EvenCursor nxt = even_next<FUSE, UNIT, W>(a, cur, wave);
+  EvenCursor nxt = even_next<FUSE, UNIT, W>(a, cur, pad, wave);
   pages = even_pages<BS, UNIT>(a, nxt);
 
   WaveState<D> st[1];
@@ -281,7 +281,7 @@ __global__ __launch_bounds__(64 * W, kEvenWavesPerCU / W) void even_decode_kerne
     constexpr int kDimThreads = D / N;
     constexpr int kSpread = acc_spread<D>();
     const EvenOut w = out_args();
-    const int tiles = even_tiles(cu.len);
+    const int tiles = even_tiles(cu.len, pad);
     const bool whole = cu.t_begin == 0 && cu.t_end == tiles;
     const int slot = 2 * share + (cu.t_begin == 0 ? 1 : 0);
     if (cu.left == 0 && threadIdx.x == 0) w.cuts[share] = even_cut(cu, tiles, whole, share, share_end, per);
@@ -342,7 +342,7 @@ __global__ __launch_bounds__(64 * W, kEvenWavesPerCU / W) void even_decode_kerne
     const bool last = even_last<W>(cur);
     const bool more = nxt.valid;
     even_load<T, BS, UNIT, D, NT>(a, nxt, pages, c, g, ahead);
-    const EvenCursor after = even_next<FUSE, UNIT, W>(a, nxt, wave);
+    const EvenCursor after = even_next<FUSE, UNIT, W>(a, nxt, pad, wave);
     pages = even_pages<BS, UNIT>(a, after);
     const int app = FUSE && cur.unit < cur.u_end ? cur.len - 1 : -1;
     if constexpr (FUSE) {

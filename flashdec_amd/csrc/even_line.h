@@ -58,8 +58,10 @@ __device__ __forceinline__ int even_row_len(const EvenArgs& a, int b) {
 }
 
 // 32-token tiles of a row; an empty row counts one (nothing in it attends, and
-// its zero output row is stored by whoever walks it)
-__device__ __forceinline__ int even_tiles(int len) { return max(1, (len + 31) >> 5); }
+// its zero output row is stored by whoever walks it).  In a short batch's line
+// (pad = min_tiles - 1, even_first) every row counts whole min_tiles, the last of
+// them without tokens.
+__device__ __forceinline__ int even_tiles(int len, int pad) { return (max(1, (len + 31) >> 5) + pad) & ~pad; }
 
 // Where a wave is on its share's line (wave-uniform).
 struct EvenCursor {
@@ -90,7 +92,7 @@ __device__ __forceinline__ bool even_last(const EvenCursor& c) {
 // The wave's next step on the line: its next unit of this segment, else the
 // next segment.
 template <bool FUSE, int UNIT, int W>
-__device__ __forceinline__ EvenCursor even_next(const EvenArgs& a, EvenCursor c, int wave) {
+__device__ __forceinline__ EvenCursor even_next(const EvenArgs& a, EvenCursor c, int pad, int wave) {
   constexpr int UPT = 32 / UNIT;
   if (c.valid && !even_last<W>(c)) {
     c.unit += W;
@@ -110,7 +112,7 @@ __device__ __forceinline__ EvenCursor even_next(const EvenArgs& a, EvenCursor c,
   }
   c.len = even_row_len<FUSE, true>(a, c.b);
   c.t_begin = 0;
-  c.t_end = min(even_tiles(c.len), c.left);
+  c.t_end = min(even_tiles(c.len, pad), c.left);
   c.left -= c.t_end;
   even_enter<UNIT, W>(c, wave);
   return c;
@@ -145,14 +147,16 @@ __device__ __forceinline__ int even_share(int block, int shares, int used) {
 // and a scan over the lanes finds the one holding the share's first tile.
 template <bool FUSE>
 __device__ __forceinline__ EvenCursor even_first(const EvenArgs& a, int block, int lane, int lane_len, int& share,
-                                                 int& per, int& share_end) {
+                                                 int& per, int& share_end, int& pad) {
   const int n = (a.num_seqs + 63) >> 6;  // rows per lane
   const int r0 = lane * n;
-  int mine = 0;
+  const int short_pad = a.min_tiles - 1;  // min_tiles is a power of two
+  int mine = 0, padded = 0;
   int len = 0;  // of the lane's row, when it has one
   if (n == 1) {
     len = lane_len;
-    mine = lane < a.num_seqs ? even_tiles(len) : 0;
+    mine = lane < a.num_seqs ? even_tiles(len, 0) : 0;
+    padded = (mine + short_pad) & ~short_pad;
   }
   for (int i = 0; n > 1 && i < n; i += 4) {
     int t[4];
@@ -160,15 +164,32 @@ __device__ __forceinline__ EvenCursor even_first(const EvenArgs& a, int block, i
     for (int j = 0; j < 4; ++j) {
       const int r = r0 + i + j;
       const bool in = i + j < n && r < a.num_seqs;
-      t[j] = even_tiles(even_row_len<FUSE, false>(a, in ? r : 0));
+      t[j] = even_tiles(even_row_len<FUSE, false>(a, in ? r : 0), 0);
       t[j] = in ? t[j] : 0;
     }
     mine += (t[0] + t[1]) + (t[2] + t[3]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) padded += (t[j] + short_pad) & ~short_pad;
   }
-  const int incl = even_scan(mine);
-  const int total = __builtin_amdgcn_readlane(incl, 63);
+  int incl = even_scan(mine);
+  int total = __builtin_amdgcn_readlane(incl, 63);
+  pad = 0;
+  // A short batch: shares of min_tiles (or twice that) end where rows do, so that
+  // no wave walks the ends of several rows one after the other and a row of one
+  // share is not cut.  The tiles without tokens take no time, and at that length
+  // there are workgroups to spare.  MI355X, graph replays, us/call as one line /
+  // with rows padded / row kernel, Hq 16, Hkv 2, tables of 2048 to 4096 tokens: 48
+  // rows of 1 .. 256 tokens 14.4 / 9.0 / 11.6, of 8 .. 2048 16.6 / 13.7 / 18.4; 100
+  // rows of 256 13.9 / 12.0 / 15.6, of 4 .. 1024 18.9 / 14.0 / 18.0.  (Up to one
+  // round of min_tiles instead of two: 9.0, 16.6, 14.1 and 18.9.)
+  if (total * a.hkv <= 2 * a.shares * a.min_tiles) {
+    pad = short_pad;
+    mine = padded;
+    incl = even_scan(mine);
+    total = __builtin_amdgcn_readlane(incl, 63);
+  }
   const int line = total * a.hkv;
-  per = max(a.min_tiles, (line + a.shares - 1) / a.shares);
+  per = (max(a.min_tiles, (line + a.shares - 1) / a.shares) + pad) & ~pad;
   EvenCursor c{};
   share = even_share(block, a.shares, (line + per - 1) / per);
   const int pos = share * per;
@@ -186,7 +207,7 @@ __device__ __forceinline__ EvenCursor even_first(const EvenArgs& a, int block, i
     const int r = l * n + i + lane;
     const bool in = i + lane < n && r < a.num_seqs;
     const int rl = even_row_len<FUSE, false>(a, in ? r : 0);
-    const int t = in ? even_tiles(rl) : 0;
+    const int t = in ? even_tiles(rl, pad) : 0;
     const int sum = even_scan(t);
     const uint64_t m = __ballot(in && at < base + sum);
     if (m) {
@@ -201,8 +222,8 @@ __device__ __forceinline__ EvenCursor even_first(const EvenArgs& a, int block, i
   c.valid = 1;
   c.b = b;
   c.len = row_len;
-  const int tiles = even_tiles(c.len);
-  c.t_begin = at - base;
+  const int tiles = even_tiles(c.len, pad);
+  c.t_begin = min(at - base, tiles);
   c.left = share_end - pos;
   c.t_end = min(tiles, c.t_begin + c.left);
   c.left -= c.t_end - c.t_begin;

@@ -147,8 +147,8 @@ Walk walk(const EvenArgs& a) {
     for (int wave = 0; wave < W; ++wave) {
       run_wave([&](int lane) {
         const int mine = lane < a.num_seqs ? length(lane) : 0;
-        int share, per, share_end;
-        EvenCursor cur = even_first<false>(a, block, lane, min(max(mine, 0), a.cap), share, per, share_end);
+        int share, per, share_end, pad;
+        EvenCursor cur = even_first<false>(a, block, lane, min(max(mine, 0), a.cap), share, per, share_end, pad);
         const bool says = lane == 0;
         if (share < 0 || share >= a.shares) fail("share out of range");
         auto write = [&](const EvenCut& c) {
@@ -167,7 +167,7 @@ Walk walk(const EvenArgs& a) {
           if (cur.unit < 0 || cur.t_begin < 0) fail("unit out of range");
           if (even_last<W>(cur)) {
             if (++segments > rows) fail("a share walks more rows than there are");
-            const int tiles = even_tiles(cur.len);
+            const int tiles = even_tiles(cur.len, pad);
             const bool whole = cur.t_begin == 0 && cur.t_end == tiles;
             if (cur.left == 0) write(even_cut(cur, tiles, whole, share, share_end, per));
             if (says && wave == 0) {
@@ -175,7 +175,7 @@ Walk walk(const EvenArgs& a) {
               if (!whole) r.slots[{cur.kvh, cur.b}].push_back(2 * share + (cur.t_begin == 0 ? 1 : 0));
             }
           }
-          cur = even_next<false, UNIT, W>(a, cur, wave);
+          cur = even_next<false, UNIT, W>(a, cur, pad, wave);
         }
       });
     }
@@ -208,7 +208,7 @@ void check_merges(const EvenArgs& a, const std::vector<EvenCut>& cuts) {
 }
 
 template <int UNIT, int W>
-void check(std::vector<int> before, std::vector<int> after, int phase_at, int hkv, int cap, int shares) {
+Walk check(std::vector<int> before, std::vector<int> after, int phase_at, int hkv, int cap, int shares) {
   g_lens[0] = before;
   g_lens[1] = after;
   g_phase_at = phase_at;
@@ -218,7 +218,7 @@ void check(std::vector<int> before, std::vector<int> after, int phase_at, int hk
   check_merges(a, w.cuts);
   for (int s = 0; s < shares; ++s)
     if (before == after && !w.written[s]) fail("a share's cut is not written");
-  if (before != after) return;
+  if (before != after) return w;
   // unchanged lengths: every tile attended once, and every cut row's parts are its merge's
   std::map<std::pair<int, int>, std::vector<int>> merged;
   for (int s = 0; s < shares; ++s) {
@@ -237,12 +237,13 @@ void check(std::vector<int> before, std::vector<int> after, int phase_at, int hk
   if (!merged.empty()) fail("a merge of a row that no share cut");
   for (int h = 0; h < hkv; ++h)
     for (int b = 0; b < rows; ++b) {
-      const int tiles = even_tiles(min(max(before[b], 0), cap));
+      const int tiles = even_tiles(min(max(before[b], 0), cap), 0);
       for (int t = 0; t < tiles; ++t) {
         const auto it = w.tiles.find({h, b, t});
         if (it == w.tiles.end() || it->second != 1) fail("a tile is not attended once");
       }
     }
+  return w;
 }
 
 }  // namespace
@@ -268,6 +269,12 @@ int main() {
         check<16, 4>(full, later, at, hkv, 960, shares);
       }
     }
+    if (rows > 100) continue;
+    // a short line: rows in shares of their own
+    const std::vector<int> few = some(rows, 150);
+    const Walk own = check<16, 8>(few, few, 1 << 30, hkv, 960, 2 * hkv * rows);
+    for (const auto& x : own.slots)
+      if (even_tiles(few[x.first.second], 0) <= 4) fail("a row of one share is cut");
   }
   // a merge's record that no workgroup of the launch wrote
   const EvenArgs a = args(5, 2, 960, 16);
