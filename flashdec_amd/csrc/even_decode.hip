@@ -550,20 +550,32 @@ extern "C" int fd_paged_decode_even_floats(const fd_paged_decode_args* args) {
 
 // The host knows what the tables hold at most, not the rows' lengths.  Against
 // the row kernel and its merge this one starts with one more round trip (the
-// lengths) and merges with one more, about 2 us a call, and saves what unequal
-// rows, tables wider than the rows, or workgroups that do not come out in whole
-// rounds cost the row kernel.  MI355X, graph replays, us/call here against the
-// row kernel (rows as long as the table / half to all of it / tables four times
-// wider):
-//   12288 tiles and more: 64 rows x 4096, Hkv 2: 46.7 / 39.2 / 39.2 against 47.1 / 45.9 / 55.6; 32 x 16384,
-//     Hkv 1: 50.5 / 41.9 / 41.9 against 47.3 / 46.8 / 57.7; 132 x 705, Hkv 4: 38.1 / 33.0 / 32.9 against
-//     48.3 / 47.9 / 60.7; 193 x 256 .. 511 of 2044, Hkv 8: 55.6 against 93.2
-//   4096 to 12288, row kernel in more than one round: 43 x 1323, Hkv 2: 17.5 / 16.7 / 16.0 against 19.2 / 22.2 /
-//     21.3; 24 x 1140, Hkv 8: 23.4 / 21.3 / 21.3 against 25.5 / 30.4 / 30.0
-//   in one round: 32 x 4096, Hkv 2: 27.5 / 25.3 against 27.0 / 27.3; 16 x 8192, Hkv 2: 28.4 / 25.2 against 25.9 /
-//     27.4; more than 448 pairs: 185 x 319, Hkv 4: 26.8 / 24.4 against 25.7 / 22.9; 16 heads per KV head (more
-//     to merge): 213 x 1290: 31.4 / 27.4 against 27.9 / 26.2; fewer than 64 pairs: 3 x 6045, Hkv 16: 30.1 / 26.0
-//     against 28.2 / 28.1
+// lengths) and merges with one more, about 2 us a call, and saves what rounds of
+// workgroups that the rows do not fill cost the row kernel.  The rows may be far
+// shorter than the tables, so a call goes here only where it gains at every
+// length.  MI355X, graph replays, us/call of the row kernel / here, Hq 16, Hkv 2
+// unless said otherwise; "mixed": lengths spread evenly over their logarithm.
+//   Row kernel in one round (pairs x splits up to the CUs): never.  Full rows
+//     gain little, rows shorter than the table lose: 8 x 2048 in 32768 9.4 /
+//     12.7, 128 x 512 in 2048 15.1 / 18.6, 64 x 4096 full 47.1 / 46.7.
+//   In more, two splits and more: always.  100 rows in 4096: x 64 12.5 / 9.7,
+//     x 512 20.8 / 18.2, mixed to 1024 18.0 / 14.0, full 82.6 / 71.5.  Under 64
+//     pairs from three rounds on: 1024 tokens in 32768, Hkv 1, 32 rows (two
+//     rounds) 14.0 / 15.1, 48 rows 19.4 / 13.3.
+//   One split: from 1024 pairs on, 2048 with more than 8 heads per KV head (more
+//     to merge).  Rows of 64 to 128, pairs: 512 11.3 / 12.3, 768 15.8 / 17.4, 1024
+//     20.5 / 19.2; Hkv 1, rows of 128 to 256: 1024 30.9 / 34.3, 2048 59.0 / 59.3.
+//   64-dim heads (half the bytes, the same fixed time): from 64 pairs, in more
+//     than three rounds, eight under four splits: 100 rows of 128 to 256, two splits
+//     (tables of 4096) 9.6 / 10.9, five (8192) 13.2 / 10.9.
+// A caller that says the lengths vary widely (balance_target) gets the balanced
+// kernel otherwise, one round whatever the lengths: from 192 pairs on.  Below, one
+// long row among short ones loses (64 pairs, 8192 in 32768: 14.3 / 16.3), and
+// mixed ones to 4096 come out even (Hq 32, Hkv 8, 128 pairs 19.1 / 20.0, 192 25.6 /
+// 24.0).
+constexpr int64_t kEvenRaggedPairs = 192;
+constexpr int64_t kEvenOneSplitPairs = 1024;
+
 extern "C" int fd_paged_decode_even_pays(const fd_paged_decode_args* args) {
   if (args == nullptr || args->struct_size != sizeof(fd_paged_decode_args))
     return set_error(FD_E_INVALID, "fd_paged_decode_even_pays: args is NULL or has another ABI's size");
@@ -571,11 +583,15 @@ extern "C" int fd_paged_decode_even_pays(const fd_paged_decode_args* args) {
   if (even_shape(a).waves == 0) return 0;
   const int64_t cap = a.max_blocks_per_seq * a.block_size;
   const int64_t pairs = a.num_seqs * a.num_kv_heads;
+  const bool many_heads = a.num_q_heads > 8 * a.num_kv_heads;
   const int64_t tiles = pairs * ((cap + 31) / 32) * a.head_dim / 128;  // of 16 KB
-  if (tiles >= 12288) return 1;
-  if (tiles < 4096 || pairs < 64 || pairs >= 448 || a.num_q_heads > 8 * a.num_kv_heads) return 0;
+  if (tiles < 12288 && (tiles < 4096 || pairs < 64 || pairs >= 448 || many_heads)) return 0;
+  if (a.balance_target > 0) return pairs >= kEvenRaggedPairs ? 1 : 0;
   const int splits = fd_paged_decode_plan(a.num_seqs, a.num_q_heads, a.num_kv_heads, a.head_dim, cap, 0);
-  return pairs * splits > device_cus() ? 1 : 0;
+  const int64_t cus = device_cus(), wgs = pairs * splits;
+  if (a.head_dim == 64) return pairs >= 64 && splits > 1 && wgs > (splits < 4 ? 8 : 3) * cus ? 1 : 0;
+  if (splits == 1) return pairs >= (many_heads ? 2 : 1) * kEvenOneSplitPairs ? 1 : 0;
+  return pairs < 64 ? wgs >= 3 * cus : wgs > cus;
 }
 
 extern "C" int fd_paged_decode_even(const fd_paged_decode_args* args, float* workspace, int64_t floats,

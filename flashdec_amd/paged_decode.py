@@ -496,19 +496,21 @@ def _decode_args(q, k_cache, v_cache, block_tables, seq_lens, out, sm_scale, blo
     args.kv_reuse = 1 if kv_reuse else 0
     if fuse_kv_append:
         _fill_append(args, append_k, append_v, slot_mapping)
+    balance = 0
+    if ragged and not use_split_kv and not fuse_kv_append and use_grouped_gqa:
+        balance = _lib.paged_decode_balance_target(num_seqs, num_kv_heads)
+    args.balance_target = balance
     args.even = 0
     # (a batch of fewer than 4096 tiles is below every line of the library's rule: no call to ask it)
     if even and not use_split_kv and num_seqs * num_kv_heads * -(-max_seq_len // 32) * head_dim >= 4096 * 128:
         floats = _lib.paged_decode_even_floats(args)
         if floats:
             args.num_splits = 1
+            args.balance_target = 0
             args.even = floats
             args.caller_workspace = False
             return args, stream
-    balance = 0
     if not use_split_kv:
-        if ragged and not fuse_kv_append and use_grouped_gqa:
-            balance = _lib.paged_decode_balance_target(num_seqs, num_kv_heads)
         if balance:
             num_splits = max(2, min(balance, -(-max_seq_len // 32)))
         else:
@@ -527,7 +529,6 @@ def _decode_args(q, k_cache, v_cache, block_tables, seq_lens, out, sm_scale, blo
         split_acc = split_max = split_sum = None
         if num_splits > 1:
             split_acc, split_max, split_sum, _ = _auto_workspace(q, num_kv_heads, num_splits, stream)
-    args.balance_target = balance
     _fill_workspace(args, split_acc, split_max, split_sum, num_splits)
     # the workspace stays alive as long as the arguments that point into it
     # (a later, larger call may replace the stream's own workspace)

@@ -326,7 +326,8 @@ int fd_paged_decode_cascade(const fd_paged_decode_args* args, const fd_cascade_a
  */
 int fd_paged_decode_even_floats(const fd_paged_decode_args* args);
 /* Whether the library would take fd_paged_decode_even for this call: 1 or 0
- * (from the shapes and what the block tables can hold; a negative FD_E* code
+ * (from the shapes and what the block tables can hold; balance_target > 0 says
+ * that the call would take balanced splits otherwise; a negative FD_E* code
  * for a NULL or foreign struct). */
 int fd_paged_decode_even_pays(const fd_paged_decode_args* args);
 int fd_paged_decode_even(const fd_paged_decode_args* args, float* workspace, int64_t floats, fd_stream_t stream);

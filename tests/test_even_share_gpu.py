@@ -139,6 +139,25 @@ def test_large_batches_take_even_shares_and_unaligned_pointers_do_not():
     assert_close_to_oracle(general, np32(out))
 
 
+@pytest.mark.parametrize(("lens", "width", "ragged", "kernel"), [
+    ([2048] * 8, 1024, False, "decode_mfma_kernel"),  # a small batch behind wide tables: one round of row workgroups
+    ([40 * i + 1 for i in range(32)], 1024, True, "decode_balanced_kernel"),  # said to be ragged, 64 pairs
+    ([40 * i + 1 for i in range(96)], 256, True, "even_decode_kernel"),  # 192 pairs
+])
+def test_calls_that_even_shares_would_slow_keep_their_kernels(lens, width, ragged, kernel):
+    import flashdec_amd as fd
+    from flashdec_amd import _lib
+
+    q, k, v, table, sl = make_paged_inputs(lens, 16, 2, 128, 32, seed=4, table_width=width)
+    _lib.record_launches(True)
+    try:
+        out = fd.decode(q, k, v, table, sl, ragged=ragged)
+        assert kernel in _lib.last_launch()[0], _lib.last_launch()
+    finally:
+        _lib.record_launches(False)
+    assert_close_to_oracle(out, _oracle(q, k, v, table, sl))
+
+
 def test_even_share_workspaces_are_a_graphs_own_and_a_threads_own():
     """A captured call's partials stay in the graph's memory whatever the stream ran before, and threads on
     one stream have a workspace each."""
