@@ -325,8 +325,10 @@ def paged_decode_attention_cascade_into(
                                (sm_scale, block_size, num_splits, prefix_splits, kv_reuse, chunk_rows, stream))
         except (AttributeError, TypeError):
             key = None  # an argument that is not a tensor: the full path raises the reference's message
-        if key is not None and last[0] == key:
-            # the previous call's metadata and settings: only data pointers change
+        if key is not None and last[0] == key and (workspace is not None
+                                                   or not torch.cuda.is_current_stream_capturing()):
+            # the previous call's metadata and settings: only data pointers
+            # change (a captured call's partials go to the graph's own memory)
             args, cas = last[1]
             args.q = q.data_ptr()
             args.k_cache = k_cache.data_ptr()
@@ -432,7 +434,8 @@ def paged_decode_attention_cascade_into(
         key = _cascade_key(q, k_cache, v_cache, block_tables, seq_lens, out, groups, workspace,
                            (sm_scale_in, block_size_in, num_splits_in, prefix_splits_in, kv_reuse, chunk_rows_in,
                             stream))
-    _LAST_CASCADE.entry = (key, (args, cas))
+    if workspace is not None or not torch.cuda.is_current_stream_capturing():
+        _LAST_CASCADE.entry = (key, (args, cas))
     return out
 
 

@@ -164,20 +164,19 @@ def _fill_append(args, append_k, append_v, slot_mapping):
 class _SplitWorkspace:
     """fp32 split partials (plus zeroed arrival counters), reused across calls.
 
-    One per (device, stream): launches on one stream are ordered.  The
-    library-chosen split path merges with the second (reducer) kernel, which
-    measured faster on MI355X than the in-launch merge (whose arrival atomics
-    serialise at the memory side); the counters are kept for callers that opt
-    into the in-launch merge and are left at zero by every launch.  Inside a
-    graph capture with no workspace yet for the capturing stream, a private
-    one is allocated for that call only.
+    The library-chosen split path merges with the second (reducer) kernel,
+    which measured faster on MI355X than the in-launch merge (whose arrival
+    atomics serialise at the memory side); the counters are kept for callers
+    that opt into the in-launch merge and are left at zero by every launch.
+    A captured call's workspace has none: their zero fill would be one more
+    node of every replay.
     """
 
     __slots__ = ("flat", "counters")
 
     def __init__(self, device, floats, counters):
         self.flat = torch.empty(floats, device=device, dtype=torch.float32)
-        self.counters = torch.zeros(counters, device=device, dtype=torch.int32)
+        self.counters = torch.zeros(counters, device=device, dtype=torch.int32) if counters else None
 
     def views(self, num_seqs, num_q_heads, num_splits, head_dim):
         # acc rows first (16-byte aligned: the kernels store and load them as
@@ -188,25 +187,30 @@ class _SplitWorkspace:
         return acc, stats[0], stats[1], self.counters
 
 
-_WORKSPACES = {}
+# Each thread's split workspaces, one per (device, stream): launches on one
+# stream are ordered, but two threads' may fall between each other's attention
+# and reducer, so they share none.  Inside a graph capture every call has a
+# workspace of its own, from the graph's memory: no later call on the stream
+# writes it between replays or frees it under them.
+_WORKSPACES = threading.local()
 
 
 def _auto_workspace(q, num_kv_heads, num_splits, stream):
     num_seqs, num_q_heads, head_dim = q.shape
     floats = num_seqs * num_q_heads * num_splits * (head_dim + 2)
+    if torch.cuda.is_current_stream_capturing():
+        return _SplitWorkspace(q.device, floats, 0).views(num_seqs, num_q_heads, num_splits, head_dim)
     counters = num_seqs * num_kv_heads * _lib.SPLIT_COUNTER_STRIDE
     key = (q.device.index, stream)
-    ws = _WORKSPACES.get(key)
+    ws = _WORKSPACES.__dict__.get(key)
     if ws is None or ws.flat.numel() < floats or ws.counters.numel() < counters:
-        if torch.cuda.is_current_stream_capturing():
-            return _SplitWorkspace(q.device, floats, counters).views(num_seqs, num_q_heads, num_splits, head_dim)
         grow = 1 if ws is None else 2
         ws = _SplitWorkspace(
             q.device,
             max(floats, grow * (ws.flat.numel() if ws else 0)),
             max(counters, grow * (ws.counters.numel() if ws else 0)),
         )
-        _WORKSPACES[key] = ws
+        _WORKSPACES.__dict__[key] = ws
     return ws.views(num_seqs, num_q_heads, num_splits, head_dim)
 
 
@@ -331,9 +335,11 @@ def paged_decode_attention_into(
                                                        num_splits, ragged, kv_reuse, stream))
         except (AttributeError, TypeError):
             key = None  # an argument that is not a tensor: the full path raises the reference's message
-    if key is not None and last[0] == key:
+    if key is not None and last[0] == key and not (last[1].library_workspace
+                                                   and torch.cuda.is_current_stream_capturing()):
         # the previous call's shapes, strides, dtypes, devices and settings:
-        # its validation and plan stand; only the data pointers change
+        # its validation and plan stand; only the data pointers change (a
+        # captured call's partials go to the graph's own memory instead)
         _, args, even = last
         _set_pointers(args, q, k_cache, v_cache, block_tables, seq_lens, out, split_kv_workspace, append_k,
                       append_v, slot_mapping)
@@ -346,7 +352,8 @@ def paged_decode_attention_into(
                               append_v, slot_mapping, (sm_scale, block_size, num_warps, kv_layout, num_stages,
                                                        num_splits, ragged, kv_reuse, stream))
         even = args.even
-        _LAST_LAUNCH.entry = (key, args, even)
+        if not (args.library_workspace and torch.cuda.is_current_stream_capturing()):
+            _LAST_LAUNCH.entry = (key, args, even)
     if not even:
         _lib.paged_decode(args, stream)
         return out
@@ -508,7 +515,7 @@ def _decode_args(q, k_cache, v_cache, block_tables, seq_lens, out, sm_scale, blo
             args.num_splits = 1
             args.balance_target = 0
             args.even = floats
-            args.caller_workspace = False
+            args.caller_workspace = args.library_workspace = False
             return args, stream
     if not use_split_kv:
         if balance:
@@ -534,6 +541,7 @@ def _decode_args(q, k_cache, v_cache, block_tables, seq_lens, out, sm_scale, blo
     # (a later, larger call may replace the stream's own workspace)
     args.workspace = (split_acc, split_max, split_sum)
     args.caller_workspace = use_split_kv
+    args.library_workspace = not use_split_kv and num_splits > 1
     return args, stream
 
 
