@@ -193,6 +193,17 @@ class _SplitWorkspace:
 # workspace of its own, from the graph's memory: no later call on the stream
 # writes it between replays or frees it under them.
 _WORKSPACES = threading.local()
+_HELD_STREAMS = 8  # whose workspaces a thread keeps, of either kind; a further stream's takes the oldest one's place
+
+
+def _hold(held, key, ws):
+    """Keeps ``ws`` for the (device, stream) ``key``.  One that is given up goes back to the allocator, which hands it
+    out on its own stream only: launches still queued there come first."""
+    held.pop(key, None)
+    while len(held) >= _HELD_STREAMS:
+        del held[next(iter(held))]
+    held[key] = ws
+    return ws
 
 
 def _auto_workspace(q, num_kv_heads, num_splits, stream):
@@ -210,7 +221,7 @@ def _auto_workspace(q, num_kv_heads, num_splits, stream):
             max(floats, grow * (ws.flat.numel() if ws else 0)),
             max(counters, grow * (ws.counters.numel() if ws else 0)),
         )
-        _WORKSPACES.__dict__[key] = ws
+        _hold(_WORKSPACES.__dict__, key, ws)
     return ws.views(num_seqs, num_q_heads, num_splits, head_dim)
 
 
@@ -229,7 +240,7 @@ def _even_workspace(device, floats, stream):
     held = _EVEN_WORKSPACES.__dict__
     ws = held.get((device.index, stream))
     if ws is None or ws.numel() < floats:
-        ws = held[(device.index, stream)] = torch.empty(floats, device=device, dtype=torch.float32)
+        ws = _hold(held, (device.index, stream), torch.empty(floats, device=device, dtype=torch.float32))
     return ws
 
 

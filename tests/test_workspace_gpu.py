@@ -74,3 +74,23 @@ def test_threads_on_one_stream_have_a_workspace_each():
     t.join()
     assert mine.data_ptr() != theirs[0].data_ptr()
     assert mine.data_ptr() == pd._auto_workspace(q, 2, 4, stream)[0].data_ptr()
+
+
+def test_a_thread_keeps_the_workspaces_of_a_few_streams_only():
+    from flashdec_amd import paged_decode as pd
+
+    q, call = _decode_call()
+    want = call()
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(3 * pd._HELD_STREAMS)]
+    outs = []
+    for _ in range(2):
+        for s in streams:
+            with torch.cuda.stream(s):
+                outs.append(call())
+                even = pd._even_workspace(q.device, 4096, s.cuda_stream)
+                assert even is pd._even_workspace(q.device, 4096, s.cuda_stream)
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, want) for o in outs)
+    for held in (pd._WORKSPACES.__dict__, pd._EVEN_WORKSPACES.__dict__):
+        assert len(held) <= pd._HELD_STREAMS and (q.device.index, streams[-1].cuda_stream) in held
