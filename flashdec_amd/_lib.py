@@ -17,7 +17,6 @@ LIB_NAME = "libflashdec_hip.so"
 LIB_PATH = Path(__file__).resolve().with_name(LIB_NAME)
 
 FD_OK = 0
-FD_E_UNSUPPORTED = -2
 FD_DTYPE_F16 = 0
 FD_DTYPE_BF16 = 1
 FD_DTYPE_F32 = 2
@@ -320,13 +319,10 @@ def paged_decode_cascade(args: PagedDecodeArgs, cascade: CascadeArgs, stream: in
 
 def paged_decode_even(args: PagedDecodeArgs, workspace: int, floats: int, stream: int) -> bool:
     """``fd_paged_decode_even``: the batch's tokens in equal shares; ``workspace`` a device pointer.
-    False where these pointers' alignment needs ``paged_decode`` (nothing was launched)."""
+    True: launched (a call that the kernel does not take raises)."""
     lib = load_library()
-    args.struct_size = ctypes.sizeof(PagedDecodeArgs)
-    rc = lib.fd_paged_decode_even(ctypes.byref(args), workspace, floats, stream)
-    if rc == FD_E_UNSUPPORTED:
-        return False
-    check(rc, "fd_paged_decode_even")
+    args.struct_size = _PAGED_DECODE_BYTES
+    check(lib.fd_paged_decode_even(ctypes.byref(args), workspace, floats, stream), "fd_paged_decode_even")
     return True
 
 

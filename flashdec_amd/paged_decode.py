@@ -346,40 +346,53 @@ def paged_decode_attention_into(
                                                        num_splits, ragged, kv_reuse, stream))
         except (AttributeError, TypeError):
             key = None  # an argument that is not a tensor: the full path raises the reference's message
-    if key is not None and last[0] == key and not (last[1].library_workspace
-                                                   and torch.cuda.is_current_stream_capturing()):
+    launch = None
+    if key is not None and last[0] == key:
+        launch = last[1]
+        if last[2] is not None:
+            launch = last[2][_off_16(q, k_cache, v_cache, append_k, append_v)]
+        if launch is not None and launch[0].library_workspace and torch.cuda.is_current_stream_capturing():
+            launch = None  # a captured call's partials go to the graph's own memory
+    if launch is not None:
         # the previous call's shapes, strides, dtypes, devices and settings:
-        # its validation and plan stand; only the data pointers change (a
-        # captured call's partials go to the graph's own memory instead)
-        _, args, even = last
+        # its validation and plan stand; only the data pointers change
+        args, even = launch
         _set_pointers(args, q, k_cache, v_cache, block_tables, seq_lens, out, split_kv_workspace, append_k,
                       append_v, slot_mapping)
     else:
         args, stream = _decode_args(q, k_cache, v_cache, block_tables, seq_lens, out, sm_scale, block_size,
                                     num_warps, kv_layout, num_stages, split_kv_workspace, num_splits, append_k,
                                     append_v, slot_mapping, ragged, kv_reuse, even=True)
-        if key is None:
-            key = _launch_key(q, k_cache, v_cache, block_tables, seq_lens, out, split_kv_workspace, append_k,
-                              append_v, slot_mapping, (sm_scale, block_size, num_warps, kv_layout, num_stages,
-                                                       num_splits, ragged, kv_reuse, stream))
         even = args.even
         if not (args.library_workspace and torch.cuda.is_current_stream_capturing()):
-            _LAST_LAUNCH.entry = (key, args, even)
-    if not even:
-        _lib.paged_decode(args, stream)
-        return out
-    ws = _even_workspace(q.device, even, stream)
-    if not _lib.paged_decode_even(args, ws.data_ptr(), even, stream):
-        # the same shapes and strides at pointers that the even-share kernel does not take
-        args, stream = _decode_args(q, k_cache, v_cache, block_tables, seq_lens, out, sm_scale, block_size,
-                                    num_warps, kv_layout, num_stages, split_kv_workspace, num_splits, append_k,
-                                    append_v, slot_mapping, ragged, kv_reuse)
+            if key is None:
+                key = _launch_key(q, k_cache, v_cache, block_tables, seq_lens, out, split_kv_workspace, append_k,
+                                  append_v, slot_mapping, (sm_scale, block_size, num_warps, kv_layout, num_stages,
+                                                           num_splits, ragged, kv_reuse, stream))
+            by_line = None
+            if args.even_asked:
+                by_line = last[2] if last is not None and last[0] == key else [None, None]
+                by_line[_off_16(q, k_cache, v_cache, append_k, append_v)] = (args, even)
+            _LAST_LAUNCH.entry = (key, (args, even), by_line)
+    if even:
+        _lib.paged_decode_even(args, _even_workspace(q.device, even, stream).data_ptr(), even, stream)
+    else:
         _lib.paged_decode(args, stream)
     return out
 
 
-# The last launch of each thread: (metadata key, PagedDecodeArgs, its even-share
-# workspace's floats).
+def _off_16(q, k_cache, v_cache, append_k, append_v):
+    """Whether a pointer that the MFMA kernels read in 16-byte pieces is not on a 16-byte line."""
+    bits = q.data_ptr() | k_cache.data_ptr() | v_cache.data_ptr()
+    if append_k is not None and append_v is not None:
+        bits |= append_k.data_ptr() | append_v.data_ptr()
+    return bits & 15 != 0
+
+
+# The last launch of each thread: (metadata key, (PagedDecodeArgs, its even-share
+# workspace's floats), None or, for shapes that the even-share rule is asked about,
+# such a pair for pointers on a 16-byte line and one for others: the rule refuses
+# the latter).
 _LAST_LAUNCH = threading.local()
 
 
@@ -520,7 +533,9 @@ def _decode_args(q, k_cache, v_cache, block_tables, seq_lens, out, sm_scale, blo
     args.balance_target = balance
     args.even = 0
     # (a batch of fewer than 4096 tiles is below every line of the library's rule: no call to ask it)
-    if even and not use_split_kv and num_seqs * num_kv_heads * -(-max_seq_len // 32) * head_dim >= 4096 * 128:
+    args.even_asked = (even and not use_split_kv
+                       and num_seqs * num_kv_heads * -(-max_seq_len // 32) * head_dim >= 4096 * 128)
+    if args.even_asked:
         floats = _lib.paged_decode_even_floats(args)
         if floats:
             args.num_splits = 1

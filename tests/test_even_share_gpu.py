@@ -139,6 +139,39 @@ def test_large_batches_take_even_shares_and_unaligned_pointers_do_not():
     assert_close_to_oracle(general, np32(out))
 
 
+def test_the_route_follows_each_calls_pointers():
+    """Calls of one shape at pointers on and off a 16-byte line, in either order and again: each takes its own kernel
+    and gives its own bits."""
+    import flashdec_amd as fd
+    from flashdec_amd import _lib
+    from flashdec_amd import paged_decode as pd
+
+    q, k, v, table, sl = make_paged_inputs([900 + 3 * i for i in range(200)], 16, 2, 128, 32, seed=6, table_width=1024)
+    shifted = torch.empty(q.numel() + 1, device=q.device, dtype=q.dtype)[1:].view(q.shape)
+    shifted.copy_(q)
+    ask = []
+    args = pd._decode_args
+
+    def counted(*a, **kw):
+        ask.append(1)
+        return args(*a, **kw)
+
+    pd._LAST_LAUNCH.__dict__.clear()
+    pd._decode_args = counted
+    _lib.record_launches(True)
+    try:
+        outs = {}
+        for query in (shifted, q, shifted, q, q, shifted):
+            out = fd.decode(query, k, v, table, sl)
+            assert any("even" in n for n in _lib.last_launch()) == (query is q)
+            assert torch.equal(out, outs.setdefault(query is q, out))
+    finally:
+        _lib.record_launches(False)
+        pd._decode_args = args
+    assert len(ask) == 2  # each prepared once
+    assert_close_to_oracle(outs[False], np32(outs[True]))
+
+
 @pytest.mark.parametrize(("lens", "width", "ragged", "kernel"), [
     ([2048] * 8, 1024, False, "decode_mfma_kernel"),  # a small batch behind wide tables: one round of row workgroups
     ([40 * i + 1 for i in range(32)], 1024, True, "decode_balanced_kernel"),  # said to be ragged, 64 pairs
