@@ -4,12 +4,12 @@ Rows attached to one registered prefix of the paged cache
 (``PagedKVCache.attach_prefix``, flashdec/cache.py:225-248) lead their block
 tables with the same physical blocks.  The reference's decode kernels read
 that prefix once per row (flashdec/kernels/paged_decode.py:330-543); the
-cascade launch reads it once per 16 (member, query head) rows of a group
-and fills all 16 columns of the MFMA tiles with them (one request of a
+cascade launch reads it once per 16, 32 or 128 (member, query head) rows of a
+group and fills all 16 columns of the MFMA tiles with them (one request of a
 GQA group of 8 fills only half):
 
-1. prefix-role workgroups attend a group's prefix for 16 of its rows each,
-   writing ``prefix_splits`` partials per row;
+1. prefix-role workgroups attend a group's prefix for one such chunk of its
+   rows each, writing ``prefix_splits`` partials per row;
 2. tail-role workgroups, in the same launch, attend every row's private
    tokens after its prefix (the whole row for rows in no group);
 3. the split reducer merges both sets of partials (log-sum-exp).
@@ -42,8 +42,9 @@ class CascadeGroups:
     prefix's block ids), ``prefix_len`` int32 ``[num_groups]`` (shared tokens,
     whole blocks), ``row_prefix_len`` int32 ``[num_seqs]`` (0 for rows in no
     group).
-    ``max_prefix_len``, ``max_tail_len`` and ``total_tail_len`` are host
-    figures for split planning.
+    ``max_prefix_len``, ``max_tail_len``, ``total_tail_len`` and
+    ``shared_tokens`` (members x prefix tokens, summed over the groups; None:
+    not known) are host figures for split planning.
     """
 
     members: torch.Tensor
@@ -52,6 +53,7 @@ class CascadeGroups:
     max_prefix_len: int
     max_tail_len: int
     total_tail_len: int
+    shared_tokens: int | None = None
 
     @property
     def num_groups(self) -> int:
@@ -130,6 +132,7 @@ def build_cascade_groups(block_tables, seq_lens, block_size, num_q_heads, num_kv
         max_prefix_len=int(prefix.max(initial=0)),
         max_tail_len=int(tails.max(initial=0)),
         total_tail_len=int(tails.sum()),
+        shared_tokens=int(row_prefix.sum(dtype=np.int64)),
     )
 
 
@@ -227,40 +230,67 @@ def plan_chunk_rows(groups, num_q_heads, num_kv_heads):
     return _lib.CASCADE_MAX_CHUNK_ROWS if rows * groups.max_prefix_len >= _WIDE_CHUNK_MIN_WORK else 16
 
 
-# plan_wide_cascade: KV heads x group rows x prefix tokens from which wide
-# prefix workgroups pay.  Same-box MI355X sweep, us/call, 16- or 32-row chunks
-# (their best) against wide ones at three quarters of the CUs, tails up to 256
-# (Hq/Hkv, sharers x prefix): above the line 16/2 24 x 16384 29.99 vs 25.70,
-# 32/4 24 x 8192 31.30 vs 25.32, 16/1 24 x 16384 26.17 vs 24.53 (6.3 M each),
-# 16/1 64 x 8192 26.01 vs 25.77 (8.4 M, the closest), 32/8 40 x 8192 51.08 vs
-# 32.55, 16/2 64 x 16384 37.08 vs 33.58; below it 16/2 40 x 8192 24.04 vs 23.38,
-# 16/1 40 x 8192 23.54 vs 24.47 (5.2 M), 16/2 24 x 4096 14.62 vs 19.06.  A wide
-# workgroup's time is its fixed part (about 8 us: launch, first loads, merge)
-# and 1.4 us for each 64 tokens.  One tail split always measured best beside
-# them, and a tail-role workgroup then outlasts the prefix role's past 512
-# tokens: 32/4 24 x 8192 34.33 vs 25.44 with tails to 512, 32.98 vs 27.20 to
-# 1024; 16/2 64 x 8192 29.29 vs 25.95, 31.85 vs 31.79; 16/2 64 x 16384 39.14 vs
-# 34.11, 40.55 vs 34.04.  Longer tails keep the 32-row chunks, which
-# tests/test_routing_gpu.py holds 64 x 16384 with tails to 700 to.
-_WIDE_TILE_MIN_WORK = 6 << 20
+# plan_wide_cascade: where wide prefix workgroups measured no slower than 16- and
+# 32-row chunks at their plan (MI355X, graph replays, tails to 512 unless said,
+# us/call old / wide; Hq/Hkv groups x sharers x prefix).  A workgroup reads its
+# range once however many of its 128 rows there are, about 1.6 us for each 64
+# tokens beside about 8 us for launch, first loads and merge, so it wants:
+#   full rows: 16/2 12 x 16 x 8192 125 / 46, 12 x 8 67 / 39, 12 x 4 42 / 37, 32 x 2
+#     51 / 74; groups of unequal sizes or prefixes count as what they leave empty
+#     (32/4, one of 40 sharers on 16384 tokens and six on 512: 156 / 201; without
+#     shared_tokens several groups keep the chunks);
+#   most of its three quarters of the CUs in use, from 8 workgroups a split on:
+#     16/1 1 x 16 x 32768 (two) 24.7 / 27.9;
+#   batches enough to pay for the fixed part: 16/2 1 x 64, 16384 (10.7 of 64
+#     tokens a workgroup) 37.2 / 34.6, 8192 (5.3) with tails to 256 26.0 / 28.2.
+#     The chunks take longer with more KV heads (32/4 1 x 24 x 8192, 5.3 batches,
+#     31.8 / 24.8; 64/4 1 x 16 with its 16 heads per KV head 24.5 / 25.6) and with
+#     many workgroups (16/2 12 x 16 x 2048, 4 batches, 48 / 31);
+#   one group's tails from 256 tokens on, or a long launch: beside short ones the
+#     chunks' plan fills whole rounds (16/2 1 x 64 x 16384, tails to 32, 34.0 / 35.1;
+#     1 x 128 x 8192 35.5 / 37.1, to 512 41.1 / 35.1).
+# Over 1200 shapes inside the rule the worst was 5 % slower, five more than 3 %.
+# Tails past 512 keep the chunks, though wide workgroups were as fast or faster up
+# to 1024 (16/2 1 x 64 x 16384 40.6 / 34.0, x 8192 31.9 / 31.8): callers hold 32-row
+# chunks at tails of 700 (tests/test_routing_gpu.py).  One tail split was best or
+# within 3 % of it.
 _WIDE_TILE_MAX_TAIL = 512
+_WIDE_TILE_TOKENS = 64  # a staged batch of a wide workgroup
 
 
 def plan_wide_cascade(num_seqs, num_q_heads, num_kv_heads, head_dim, groups, num_cus):
     """(prefix splits, tail splits) of a launch with wide prefix workgroups
     (``CASCADE_WIDE_CHUNK_ROWS`` rows each) on three quarters of the CUs, the tails' on the rest, or
     None for 16- and 32-row chunks."""
-    if groups.max_tail_len > _WIDE_TILE_MAX_TAIL:
+    if head_dim != 128 or groups.max_tail_len > _WIDE_TILE_MAX_TAIL:
         return None
-    if num_seqs * num_q_heads * groups.max_prefix_len < _WIDE_TILE_MIN_WORK:
-        return None  # fewer rows than that in all: no look at the index tensors' shapes
-    rows = groups.max_members * (num_q_heads // num_kv_heads)
-    if head_dim != 128 or groups.num_groups * num_kv_heads * rows * groups.max_prefix_len < _WIDE_TILE_MIN_WORK:
+    # (too few rows for half a chunk in all: no look at the index tensors' shapes)
+    if 2 * num_seqs * num_q_heads < num_kv_heads * _lib.CASCADE_WIDE_CHUNK_ROWS:
         return None
-    units = groups.num_groups * num_kv_heads * prefix_chunks(groups, num_q_heads, num_kv_heads,
-                                                             _lib.CASCADE_WIDE_CHUNK_ROWS)
+    num_groups, members, group = groups.num_groups, groups.max_members, num_q_heads // num_kv_heads
+    wide_rows = _lib.CASCADE_WIDE_CHUNK_ROWS
+    chunks = prefix_chunks(groups, num_q_heads, num_kv_heads, wide_rows)
+    units = num_groups * num_kv_heads * chunks
+    many = num_groups > 1
+    if units < 8 or many and groups.shared_tokens is None:
+        return None
     tiles = -(-groups.max_prefix_len // 32)
-    return max(1, min(num_cus * 3 // (4 * units), tiles // 4, 1024)), 1
+    splits = max(1, min(num_cus * 3 // (4 * units), tiles // 4, 1024))
+    if 8 * units * splits < 5 * num_cus:
+        return None
+    batches = 32 * tiles / (_WIDE_TILE_TOKENS * splits)
+    rows = members * group
+    if many:
+        # share of the launch's rows x prefix tokens that is there
+        filled = groups.shared_tokens * group / (num_groups * chunks * wide_rows * groups.max_prefix_len)
+        pays = filled >= 0.85 and batches >= (4 if units >= 24 else 8)
+        if chunks == 1 and 2 * rows >= wide_rows and units >= 12 and batches >= 8:
+            pays = pays or filled >= 0.75 * rows / wide_rows
+    else:
+        pays = (4 * rows >= 3 * chunks * wide_rows
+                and batches >= (5 if num_kv_heads >= 4 and group <= 8 else 8)
+                and (num_kv_heads >= 8 or groups.max_tail_len >= 256 or units >= 16 and batches >= 16))
+    return (splits, 1) if pays else None
 
 
 def prefix_chunks(groups, num_q_heads, num_kv_heads, chunk_rows=16):
@@ -450,7 +480,7 @@ def _cascade_key(q, k_cache, v_cache, block_tables, seq_lens, out, groups, works
         return (t.shape, t.stride(), t.dtype, t.device)
 
     figures = (groups.num_groups, groups.max_members, groups.max_prefix_len, groups.max_tail_len,
-               groups.total_tail_len, meta(groups.members), meta(groups.prefix_len), meta(groups.row_prefix_len))
+               groups.total_tail_len, groups.shared_tokens, meta(groups.members), meta(groups.prefix_len), meta(groups.row_prefix_len))
     return (_launch_key(q, k_cache, v_cache, block_tables, seq_lens, out, workspace, None, None, None, settings),
             figures)
 

@@ -478,7 +478,8 @@ class DecodeEngine:
             self._cascade_cache = (key, CascadeGroups(members=members.to(dev), prefix_len=prefix.to(dev),
                                                       row_prefix_len=row_prefix.to(dev),
                                                       max_prefix_len=int(prefix.max()), max_tail_len=0,
-                                                      total_tail_len=0), row_prefix.tolist())
+                                                      total_tail_len=0, shared_tokens=int(row_prefix.sum())),
+                                   row_prefix.tolist())
         _, cached, row_prefix = self._cascade_cache
         tails = [max(0, n + 1 - p) for n, p in zip(lengths, row_prefix)]  # the new token included
         return dataclasses.replace(cached, max_tail_len=max(tails), total_tail_len=sum(tails))

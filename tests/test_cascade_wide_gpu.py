@@ -69,6 +69,23 @@ def test_wide_chunks_are_no_further_from_64_bits_than_32_row_chunks(heads, share
     assert off[0] <= off[1], off
 
 
+@pytest.mark.parametrize(("kv_reuse", "nt"), [(True, "false"), (False, "true")])
+@pytest.mark.parametrize(("heads", "groups", "sharers", "blocks"), [((32, 8), 1, 24, 256), ((16, 2), 12, 16, 64)])
+def test_the_rule_reaches_the_wide_kernel(heads, groups, sharers, blocks, kv_reuse, nt):
+    hq, hkv = heads
+    q, k, v, table, lens, _ = make_prefix_inputs([(blocks, [(29 * i) % 300 + 1 for i in range(sharers)])] * groups,
+                                                 [40], hq, hkv, 32, torch.bfloat16)
+    g = cascade.build_cascade_groups(table, lens, 32, hq, hkv)
+    _lib.record_launches(True)
+    try:
+        out = cascade.paged_decode_attention_cascade(q, k, v, table, lens, groups=g, kv_reuse=kv_reuse)
+        assert _lib.last_launch()[0] == f"fd::cascade_wide_kernel<__bf16, 32, {nt}>", _lib.last_launch()
+    finally:
+        _lib.record_launches(False)
+    assert torch.equal(out, cascade.paged_decode_attention_cascade(q, k, v, table, lens, groups=g, kv_reuse=kv_reuse))
+    assert_close_to_oracle(out, _oracle(q, k, v, table, lens))
+
+
 def test_plan_and_explicit_settings():
     def groups(members, prefix, tail=512):
         return cascade.CascadeGroups(members=torch.zeros((1, members), dtype=torch.int32),
