@@ -1129,9 +1129,10 @@ __global__ __launch_bounds__(64 * waves_for<UNIT>(), 1) void cascade_decode_kern
 // two column blocks by two token groups.  The chunks of one split are
 // consecutive and share an XCD's L2 (xcd_blocks).  Bound by the issue of a
 // batch's phases one after the other (two waves a SIMD, one barrier a batch:
-// 1.4 us per 64 tokens, of which 0.5 are matrix products, 0.6 vector
-// instructions and 0.4 LDS reads).  64 rows on a 16384-token prefix, Hq 16 /
-// Hkv 2: 37.1 -> 33.6 us a call; 40 on 8192, Hq 32 / Hkv 8: 51.1 -> 32.6.
+// 1.6 us per 64 tokens, of which 0.5 are matrix products, 0.8 vector
+// instructions, the exact maximum's rescales among them, and 0.4 LDS reads).  64
+// rows on a 16384-token prefix with tails to 512, Hq 16 / Hkv 2: 37.2 -> 34.6 us a
+// call; 40 on 8192, Hq 32 / Hkv 8: 59.3 -> 35.0.
 constexpr int kPrefixRowGroups = 4;
 using PrefixShape = WideShape<128, kPrefixMaxColBlocks, kPrefixRowGroups, 2>;
 static_assert(PrefixShape::kRows == FD_CASCADE_WIDE_CHUNK_ROWS && PrefixShape::kWaves == kMaxWaves);
@@ -1183,8 +1184,8 @@ __global__ __launch_bounds__(64 * kMaxWaves, 1) void cascade_wide_kernel(
   int t0, t1;
   split_tiles(prefix_splits, split, eff, 0, t0, t1);
   const WideWork w{lead_ok ? lead : 0, gk % hkv, 32 * t0, static_cast<int>(min<int64_t>(32 * t1, eff))};
-  wide_attend<T, BS, 128, RB, kPrefixRowGroups, 2, false>(p, w, col_b, col_h, col_ok, p.splits + split,
-                                                          *reinterpret_cast<Lds*>(raw));
+  wide_attend<T, BS, 128, RB, kPrefixRowGroups, 2>(p, w, col_b, col_h, col_ok, p.splits + split,
+                                                   *reinterpret_cast<Lds*>(raw));
 }
 
 // ====================================================== generic path ====

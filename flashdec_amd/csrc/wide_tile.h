@@ -1,10 +1,10 @@
 // Device code of the wide decode workgroup: many query rows on one read of a
 // K/V range.  A group that shares a prefix brings hundreds of (member, head)
-// rows to the same tokens, and a KV head may serve more query heads than two
-// MFMA column blocks hold.  The row kernels keep a wave's K/V unit in its
+// rows to the same tokens.  The row kernels keep a wave's K/V unit in its
 // registers, so every 32 of those rows read the tokens again; here the
 // workgroup stages a batch of tokens in LDS once and each wave attends it with
-// its own rows.
+// its own rows.  (The range is read again by the group's other chunks: plain
+// loads.)
 #pragma once
 
 #include "decode_unit.h"
@@ -27,7 +27,8 @@ struct WideShape {
   static constexpr int kRun = 8;
   static constexpr int kRuns = kTokens / kRun;
   static constexpr int kLoads = kRun / kLoadRows;  // of K, and as many of V
-  static_assert(kWaves >= kRuns, "a run for each of the first kRuns waves");
+  static_assert(kWaves == kRuns, "a run for each wave");
+  static_assert(D == 128, "the tiles' swizzle");
   static constexpr int kTileBytes = kTokens * D * 2;
   static constexpr int kMergeBytes = (TG - 1) * kRows * D * 4;
   static constexpr int kStageBytes = 4 * kTileBytes > kMergeBytes ? 4 * kTileBytes : kMergeBytes;
@@ -50,7 +51,7 @@ __device__ __forceinline__ int wide_k_at(int row, int piece) {
 }
 template <int D>
 __device__ __forceinline__ int wide_v_at(int row, int pair) {
-  return row * (2 * D) + ((pair ^ (D == 128 ? row & 7 : (row >> 1) & 3)) << 5);
+  return row * (2 * D) + ((pair ^ (row & 7)) << 5);
 }
 
 // Four rows of the lane's 16-lane group, transposed: the lane gives the address
@@ -73,10 +74,10 @@ struct WideRegs {
   u32x4 k[S::kLoads], v[S::kLoads];
 };
 
-// First token of the wave's run; past the range for the waves without one.
+// First token of the wave's run.
 template <typename S>
 __device__ __forceinline__ int wide_run(const WideWork& w, int batch, int wave) {
-  return S::kWaves > S::kRuns && wave >= S::kRuns ? w.limit : w.begin + batch * S::kTokens + wave * S::kRun;
+  return w.begin + batch * S::kTokens + wave * S::kRun;
 }
 
 template <typename S, int BS>
@@ -105,7 +106,7 @@ __device__ __forceinline__ int wide_live(const DecodeParams& p, const WideWork& 
 // an invalid block, goes through empty descriptors: zeros and no read), so
 // that the number in flight is the same on every path and the wait for a batch
 // leaves the next one's loads in flight.
-template <typename T, typename S, int BS, bool NT>
+template <typename S, int BS>
 __device__ __forceinline__ void wide_load(const DecodeParams& p, const WideWork& w, int batch, int wave, int lane,
                                           int32_t page, WideRegs<S>& r) {
   const int tok = wide_run<S>(w, batch, wave);
@@ -121,11 +122,11 @@ __device__ __forceinline__ void wide_load(const DecodeParams& p, const WideWork&
 #pragma unroll
   for (int j = 0; j < S::kLoads; ++j)
     r.k[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                           kr, row * ks2 + piece, (row0 + j * S::kLoadRows) * ks2, NT ? 2 : 0));
+                                           kr, row * ks2 + piece, (row0 + j * S::kLoadRows) * ks2, 0));
 #pragma unroll
   for (int j = 0; j < S::kLoads; ++j)
     r.v[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                           vr, row * vs2 + piece, (row0 + j * S::kLoadRows) * vs2, NT ? 2 : 0));
+                                           vr, row * vs2 + piece, (row0 + j * S::kLoadRows) * vs2, 0));
 }
 
 // A batch's rows into its LDS tiles.  Rows past the attended tokens are stored
@@ -133,7 +134,6 @@ __device__ __forceinline__ void wide_load(const DecodeParams& p, const WideWork&
 template <typename S, int D>
 __device__ __forceinline__ void wide_stage(const DecodeParams& p, const WideWork& w, int batch, int wave, int lane,
                                            int32_t page, const WideRegs<S>& r, WideLds<S>& lds, int buf) {
-  if (S::kWaves > S::kRuns && wave >= S::kRuns) return;
   uint8_t* kt = lds.stage + buf * 2 * S::kTileBytes;
   const int live = wide_live<S>(p, w, wide_run<S>(w, batch, wave), page);
   const int row = lane / S::kPieces, piece = lane % S::kPieces;
@@ -219,7 +219,7 @@ __device__ __forceinline__ void wide_compute(const u32x4 (&qf)[RB][D / 32], floa
 
 // The whole workgroup: rows (col_b, col_h) of every column, the range w, and
 // the workspace split that takes the partials.
-template <typename T, int BS, int D, int RB, int RG, int TG, bool NT>
+template <typename T, int BS, int D, int RB, int RG, int TG>
 __device__ __forceinline__ void wide_attend(const DecodeParams& p, const WideWork& w, const int (&col_b)[RB],
                                             const int (&col_h)[RB], const bool (&col_ok)[RB], int ws,
                                             WideLds<WideShape<D, RB, RG, TG>>& lds) {
@@ -235,8 +235,8 @@ __device__ __forceinline__ void wide_attend(const DecodeParams& p, const WideWor
   int32_t page_b = wide_page<S, BS>(p, w, 1, wave);
   int32_t next = wide_page<S, BS>(p, w, 2, wave);
   WideRegs<S> ra, rb;
-  wide_load<T, S, BS, NT>(p, w, 0, wave, lane, page_a, ra);
-  wide_load<T, S, BS, NT>(p, w, 1, wave, lane, page_b, rb);
+  wide_load<S, BS>(p, w, 0, wave, lane, page_a, ra);
+  wide_load<S, BS>(p, w, 1, wave, lane, page_b, rb);
   __builtin_amdgcn_sched_barrier(0);  // ahead of the rows' own loads and their wait
   u32x4 qf[RB][KS];
 #pragma unroll
@@ -268,7 +268,7 @@ __device__ __forceinline__ void wide_attend(const DecodeParams& p, const WideWor
     wide_stage<S, D>(p, w, i, wave, lane, page, r, lds, buf);
     page = next;
     next = after;
-    wide_load<T, S, BS, NT>(p, w, i + 2, wave, lane, page, r);
+    wide_load<S, BS>(p, w, i + 2, wave, lane, page, r);
     __syncthreads();
     if (i < batches) wide_compute<T, S, D, RB>(qf, p.scale_log2, tg, c, g, lds, buf, st);
     ++i;
