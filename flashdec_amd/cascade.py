@@ -238,7 +238,8 @@ def plan_chunk_rows(groups, num_q_heads, num_kv_heads):
 #   full rows: 16/2 12 x 16 x 8192 125 / 46, 12 x 8 67 / 39, 12 x 4 42 / 37, 32 x 2
 #     51 / 74; groups of unequal sizes or prefixes count as what they leave empty
 #     (32/4, one of 40 sharers on 16384 tokens and six on 512: 156 / 201; without
-#     shared_tokens several groups keep the chunks);
+#     shared_tokens several groups keep the chunks).  From eight KV heads on half
+#     full does, the chunks' launches being longer there (32/8 1 x 40 x 8192 59 / 35);
 #   most of its three quarters of the CUs in use, from 8 workgroups a split on:
 #     16/1 1 x 16 x 32768 (two) 24.7 / 27.9;
 #   batches enough to pay for the fixed part: 16/2 1 x 64, 16384 (10.7 of 64
@@ -287,7 +288,8 @@ def plan_wide_cascade(num_seqs, num_q_heads, num_kv_heads, head_dim, groups, num
         if chunks == 1 and 2 * rows >= wide_rows and units >= 12 and batches >= 8:
             pays = pays or filled >= 0.75 * rows / wide_rows
     else:
-        pays = (4 * rows >= 3 * chunks * wide_rows
+        quarters = 2 if num_kv_heads >= 8 and units >= 12 and batches >= 8 else 3
+        pays = (4 * rows >= quarters * chunks * wide_rows
                 and batches >= (5 if num_kv_heads >= 4 and group <= 8 else 8)
                 and (num_kv_heads >= 8 or groups.max_tail_len >= 256 or units >= 16 and batches >= 16))
     return (splits, 1) if pays else None

@@ -32,6 +32,7 @@ def _plan(hq, hkv, sizes, prefixes, tail=512, known=True, head_dim=128):
     (16, 1, [16], 32768),       # two workgroups a split
     (16, 2, [64], 8192, 256),   # 5.3 batches
     (64, 4, [16], 8192),
+    (32, 4, [33], 16384),       # 264 of 384 rows
     (16, 2, [64], 16384, 32),   # short tails
     (16, 2, [64], 16384, 513),  # long ones
     (8, 8, [24], 32768),        # 24 of 128 rows
@@ -44,6 +45,7 @@ def test_launches_that_lose_keep_the_chunks(case):
     ((16, 2, [64], 16384), (24, 1)),
     ((32, 4, [24], 8192), (24, 1)),
     ((32, 8, [24], 8192, 32), (24, 1)),
+    ((32, 8, [40], 8192), (12, 1)),      # 160 of 256 rows, eight KV heads
     ((16, 2, [16] * 12, 8192), (8, 1)),
     ((16, 2, [8] * 12, 8192), (8, 1)),   # half the rows of one chunk
     ((16, 2, [16] * 12, 2048), (8, 1)),  # 24 workgroups a split, 4 batches
