@@ -3,8 +3,8 @@
 Mirrors cysong2025/flashdec ``flashdec/_fused_rope_kv_append.py``:
 
 * :func:`fused_rope_kv_append` (:210-258) -- checked public primitive; it
-  validates structure, then index *values* with device reductions that sync
-  (:128-145), then launches.
+  validates structure, then index *values* (:128-145, reductions there; one
+  launch and a wait for it here), then launches.
 * :func:`_fused_rope_kv_append_trusted` (:261-309) -- for cache-owned
   transaction metadata: same structural checks, no value reductions, int64
   indices required.

@@ -158,3 +158,20 @@ def test_noalloc_rejects_a_workspace_and_oversized_launches_before_any_hip_call(
     assert lib.fd_paged_decode_noalloc(ctypes.byref(args), None) == -1
     assert b"struct_size" in lib.fd_last_error()
     assert lib.fd_paged_decode_noalloc(None, None) == -1
+
+
+@pytest.mark.skipif(shutil.which("gcc") is None, reason="gcc not available")
+def test_index_check_struct_matches_c_layout(tmp_path):
+    src = tmp_path / "probe.c"
+    fields = [name for name, _ in _lib.IndexCheckArgs._fields_]
+    src.write_text('#include <stddef.h>\n#include <stdio.h>\n#include "flashdec_hip.h"\nint main(void) {\n'
+                   '  printf("%zu\\n", sizeof(fd_index_check_args));\n'
+                   + "".join(f'  printf("%zu\\n", offsetof(fd_index_check_args, {f}));\n' for f in fields)
+                   + "  return 0;\n}\n")
+    exe = tmp_path / "probe"
+    subprocess.run(["gcc", "-std=c11", "-Wall", "-Werror", "-I", str(HEADER.parent), str(src), "-o", str(exe)],
+                   check=True)
+    got = [int(x) for x in subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split()]
+    assert got == [ctypes.sizeof(_lib.IndexCheckArgs)] + [getattr(_lib.IndexCheckArgs, f).offset for f in fields]
+    consts = dict(re.findall(r"#define\s+(FD_\w+)\s+\(?(-?\d+)\)?", HEADER.read_text()))
+    assert int(consts["FD_CASCADE_WIDE_CHUNK_ROWS"]) == _lib.CASCADE_WIDE_CHUNK_ROWS

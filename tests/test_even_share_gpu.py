@@ -21,12 +21,12 @@ from tests.helpers import assert_close_to_oracle, make_paged_inputs, np32
 pytestmark = pytest.mark.gpu
 
 
-def _even(q, k, v, table, lens, out, append=(None, None, None)):
+def _even(q, k, v, table, lens, out, append=(None, None, None), kv_reuse=False):
     from flashdec_amd import _lib
     from flashdec_amd.paged_decode import _decode_args
 
     args, stream = _decode_args(q, k, v, table, lens, out, None, None, 2, "token_major", None, None, 1, *append,
-                                False, False)
+                                False, kv_reuse)
     args.num_splits = 1
     args.struct_size = ctypes.sizeof(_lib.PagedDecodeArgs)
     floats = _lib.load_library().fd_paged_decode_even_floats(ctypes.byref(args))
@@ -90,6 +90,55 @@ def test_even_shares_on_views_wide_tables_and_bad_blocks(block_size):
 
     plain = paged_decode_attention(q, k, v, table, sl)  # the row kernel at this size
     assert_close_to_oracle(want, np32(plain))
+
+
+@pytest.mark.parametrize("lens", [[int(x) for x in np.random.default_rng(9).integers(0, 70, 4200)],
+                                  [0] * 4133 + [33] * 3 + [0] * 64 + [5000]])
+def test_even_shares_of_more_rows_than_one_search_pass_sees(lens):
+    """More than 64 rows a lane: the row search carries its base from one pass to the next."""
+    q, k, v, table, sl = make_paged_inputs(lens, 4, 1, 128, 16, seed=12)
+    out = _even(q, k, v, table, sl, torch.full_like(q, 7.0))
+    assert_close_to_oracle(out, _oracle(q, k, v, table, sl))
+    assert torch.count_nonzero(out[sl == 0]) == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("block_size", [8, 16, 32])
+@pytest.mark.parametrize(("hq", "hkv", "d", "lens"), [(16, 2, 128, EDGES), (14, 2, 64, EDGES), (8, 4, 128, MANY),
+                                                      (8, 1, 64, MANY)])
+def test_even_shares_with_cached_loads_and_an_unaligned_output(hq, hkv, d, lens, block_size, dtype):
+    """Rows may share blocks; an output one element past a 16-byte line takes the rows' stores all the same."""
+    q, k, v, table, sl = make_paged_inputs(lens, hq, hkv, d, block_size, dtype, seed=block_size + d)
+    flat = torch.full((q.numel() + 8,), 7.0, device=q.device, dtype=dtype)
+    out = flat[1 : 1 + q.numel()].view(q.shape)
+    assert out.data_ptr() % 16
+    want = _even(q, k, v, table, sl, torch.empty_like(q))
+    assert torch.equal(_even(q, k, v, table, sl, out, kv_reuse=True), want)
+    assert flat[0] == 7.0 and bool((flat[1 + q.numel() :] == 7.0).all())
+
+
+def test_even_shares_append_into_8_token_blocks():
+    """The C ABI takes them (the Python call's grouped rule does not)."""
+    from flashdec_amd import _lib
+    from flashdec_amd import paged_decode as pd
+
+    lens = [1, 9, 64, 200, 777]
+    q, k, v, table, sl = make_paged_inputs(lens, 16, 2, 128, 8, seed=8)
+    ak, av = (torch.randn((len(lens), 2, 128), device="cuda").to(q.dtype) for _ in range(2))
+    pos = sl.long() - 1
+    slots = table.long().gather(1, (pos // 8)[:, None])[:, 0] * 8 + pos % 8
+    k1, v1, out = k.clone(), v.clone(), torch.empty_like(q)
+    args, stream = pd._decode_args(q, k1, v1, table, sl, out, None, None, 2, "token_major", None, None, 1, None, None,
+                                   None, False, False)
+    args.num_splits = 1
+    pd._fill_append(args, ak, av, slots)
+    args.struct_size = ctypes.sizeof(_lib.PagedDecodeArgs)
+    floats = _lib.load_library().fd_paged_decode_even_floats(ctypes.byref(args))
+    ws = torch.full((floats,), float("nan"), device=q.device)
+    assert _lib.paged_decode_even(args, ws.data_ptr(), floats, stream)
+    k[slots // 8, :, slots % 8], v[slots // 8, :, slots % 8] = ak, av
+    assert torch.equal(k1, k) and torch.equal(v1, v)
+    assert_close_to_oracle(out, _oracle(q, k, v, table, sl))
 
 
 @pytest.mark.parametrize("block_size", [16, 32])
