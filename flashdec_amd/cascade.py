@@ -252,9 +252,9 @@ def plan_chunk_rows(groups, num_q_heads, num_kv_heads):
 #     1 x 128 x 8192 35.5 / 37.1, to 512 41.1 / 35.1).
 # Over 1200 shapes inside the rule the worst was 5 % slower, five more than 3 %.
 # Tails past 512 keep the chunks, though wide workgroups were as fast or faster up
-# to 1024 (16/2 1 x 64 x 16384 40.6 / 34.0, x 8192 31.9 / 31.8): callers hold 32-row
+# to 1024 (16/2 1 x 64 x 16384 40.5 / 35.7, x 8192 30.5 / 30.1): callers hold 32-row
 # chunks at tails of 700 (tests/test_routing_gpu.py).  One tail split was best or
-# within 3 % of it.
+# within 2 % of it.
 _WIDE_TILE_MAX_TAIL = 512
 _WIDE_TILE_TOKENS = 64  # a staged batch of a wide workgroup
 
