@@ -329,8 +329,8 @@ def paged_decode_even(args: PagedDecodeArgs, workspace: int, floats: int, stream
 def paged_decode_even_floats(args: PagedDecodeArgs) -> int:
     """fp32 words of workspace that ``paged_decode_even`` needs for this call where the library would
     take it, else 0."""
-    lib = load_library()
-    args.struct_size = ctypes.sizeof(PagedDecodeArgs)
+    lib = _lib or load_library()
+    args.struct_size = _PAGED_DECODE_BYTES
     pays = lib.fd_paged_decode_even_pays(ctypes.byref(args))
     if pays < 0:
         check(pays, "fd_paged_decode_even_pays")
@@ -338,7 +338,7 @@ def paged_decode_even_floats(args: PagedDecodeArgs) -> int:
 
 
 def paged_decode_plan(num_seqs, num_q_heads, num_kv_heads, head_dim, max_seq_len, total_seq_len=0) -> int:
-    lib = load_library()
+    lib = _lib or load_library()
     rc = lib.fd_paged_decode_plan(num_seqs, num_q_heads, num_kv_heads, head_dim, max_seq_len, total_seq_len)
     if rc < 0:
         check(rc, "fd_paged_decode_plan")

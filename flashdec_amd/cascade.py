@@ -426,8 +426,10 @@ def paged_decode_attention_cascade_into(
         if isinstance(v, bool) or not isinstance(v, int) or v <= 0:
             raise ValueError(f"{name} must be a positive integer")
     stream = _lib.current_stream_handle(q.device)
+    captured = False
     if workspace is None:
-        acc, mx, sm, _ = _auto_workspace(q, num_kv_heads, num_splits + prefix_splits, stream)
+        acc, mx, sm, counters = _auto_workspace(q, num_kv_heads, num_splits + prefix_splits, stream)
+        captured = counters is None  # the workspace is a graph's own
     else:
         acc, mx, sm = workspace
         need = num_splits + prefix_splits
@@ -466,7 +468,7 @@ def paged_decode_attention_cascade_into(
         key = _cascade_key(q, k_cache, v_cache, block_tables, seq_lens, out, groups, workspace,
                            (sm_scale_in, block_size_in, num_splits_in, prefix_splits_in, kv_reuse, chunk_rows_in,
                             stream))
-    if workspace is not None or not torch.cuda.is_current_stream_capturing():
+    if not captured:
         _LAST_CASCADE.entry = (key, (args, cas))
     return out
 

@@ -181,10 +181,13 @@ class _SplitWorkspace:
     def views(self, num_seqs, num_q_heads, num_splits, head_dim):
         # acc rows first (16-byte aligned: the kernels store and load them as
         # float4), then max and sum as two [B, Hq, S] planes with equal strides
-        rows = num_seqs * num_q_heads * num_splits
-        acc = self.flat[: rows * head_dim].view(num_seqs, num_q_heads, num_splits, head_dim)
-        stats = self.flat[rows * head_dim : rows * (head_dim + 2)].view(2, num_seqs, num_q_heads, num_splits)
-        return acc, stats[0], stats[1], self.counters
+        # (one tensor operation each: half the host time of slices and views)
+        per = num_q_heads * num_splits
+        acc = self.flat.as_strided((num_seqs, num_q_heads, num_splits, head_dim),
+                                   (per * head_dim, num_splits * head_dim, head_dim, 1), 0)
+        shape, strides, at = (num_seqs, num_q_heads, num_splits), (per, num_splits, 1), num_seqs * per * head_dim
+        return (acc, self.flat.as_strided(shape, strides, at), self.flat.as_strided(shape, strides, at + num_seqs * per),
+                self.counters)
 
 
 # Each thread's split workspaces, one per (device, stream): launches on one
@@ -364,7 +367,7 @@ def paged_decode_attention_into(
                                     num_warps, kv_layout, num_stages, split_kv_workspace, num_splits, append_k,
                                     append_v, slot_mapping, ragged, kv_reuse, even=True)
         even = args.even
-        if not (args.library_workspace and torch.cuda.is_current_stream_capturing()):
+        if not args.captured_workspace:
             if key is None:
                 key = _launch_key(q, k_cache, v_cache, block_tables, seq_lens, out, split_kv_workspace, append_k,
                                   append_v, slot_mapping, (sm_scale, block_size, num_warps, kv_layout, num_stages,
@@ -532,16 +535,19 @@ def _decode_args(q, k_cache, v_cache, block_tables, seq_lens, out, sm_scale, blo
         balance = _lib.paged_decode_balance_target(num_seqs, num_kv_heads)
     args.balance_target = balance
     args.even = 0
-    # (a batch of fewer than 4096 tiles is below every line of the library's rule: no call to ask it)
+    # (no call to ask the library's rule about a batch of fewer than 4096 tiles, below every line of it, a layout or
+    # group that the kernel does not take, or 64-dim heads in few pairs)
     args.even_asked = (even and not use_split_kv
-                       and num_seqs * num_kv_heads * -(-max_seq_len // 32) * head_dim >= 4096 * 128)
+                       and num_seqs * num_kv_heads * -(-max_seq_len // 32) * head_dim >= 4096 * 128
+                       and kv_layout == "token_major" and group_size <= 16
+                       and (head_dim == 128 or num_seqs * num_kv_heads >= 64))
     if args.even_asked:
         floats = _lib.paged_decode_even_floats(args)
         if floats:
             args.num_splits = 1
             args.balance_target = 0
             args.even = floats
-            args.caller_workspace = args.library_workspace = False
+            args.caller_workspace = args.library_workspace = args.captured_workspace = False
             return args, stream
     if not use_split_kv:
         if balance:
@@ -561,13 +567,14 @@ def _decode_args(q, k_cache, v_cache, block_tables, seq_lens, out, sm_scale, blo
                 num_splits = max(1, min(8 * num_splits, -(-max_seq_len // 64), 4096))
         split_acc = split_max = split_sum = None
         if num_splits > 1:
-            split_acc, split_max, split_sum, _ = _auto_workspace(q, num_kv_heads, num_splits, stream)
+            split_acc, split_max, split_sum, counters = _auto_workspace(q, num_kv_heads, num_splits, stream)
     _fill_workspace(args, split_acc, split_max, split_sum, num_splits)
     # the workspace stays alive as long as the arguments that point into it
     # (a later, larger call may replace the stream's own workspace)
     args.workspace = (split_acc, split_max, split_sum)
     args.caller_workspace = use_split_kv
     args.library_workspace = not use_split_kv and num_splits > 1
+    args.captured_workspace = args.library_workspace and counters is None  # a graph's own
     return args, stream
 
 

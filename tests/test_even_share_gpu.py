@@ -240,6 +240,27 @@ def test_calls_that_even_shares_would_slow_keep_their_kernels(lens, width, ragge
     assert_close_to_oracle(out, _oracle(q, k, v, table, sl))
 
 
+def test_the_rule_is_asked_only_where_it_can_take_a_call(monkeypatch):
+    """Each new shape pays for the question: none for layouts, groups and sizes that are below every line."""
+    from flashdec_amd import _lib
+    from flashdec_amd import paged_decode as pd
+
+    asked = []
+    monkeypatch.setattr(_lib, "paged_decode_even_floats", lambda args: asked.append(args.num_seqs) or 0)
+    for hq, hkv, d, batch, width, layout, times in [(16, 2, 128, 100, 128, "token_major", 1),
+                                                    (16, 2, 128, 100, 128, "dim_major", 0),
+                                                    (71, 1, 64, 300, 128, "token_major", 0),
+                                                    (14, 2, 64, 20, 1024, "token_major", 0),
+                                                    (16, 2, 128, 16, 64, "token_major", 0)]:
+        q, k, v, table, sl = make_paged_inputs([40] * batch, hq, hkv, d, 32, seed=1, table_width=width,
+                                               kv_layout=layout)
+        asked.clear()
+        out = pd.paged_decode_attention(q, k, v, table, sl, kv_layout=layout)
+        assert len(asked) == times
+        want = oracle_decode(np32(q), np32(k), np32(v), table.cpu().numpy(), sl.cpu().numpy(), kv_layout=layout)
+        assert_close_to_oracle(out, want)
+
+
 def test_even_share_workspaces_are_a_graphs_own_and_a_threads_own():
     """A captured call's partials stay in the graph's memory whatever the stream ran before, and threads on
     one stream have a workspace each."""
