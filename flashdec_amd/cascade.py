@@ -30,7 +30,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .paged_decode import (_auto_workspace, _cache_strides, _fill_common, _fill_workspace, _launch_key,
+from .paged_decode import (_auto_workspace, _cache_strides, _capturing, _fill_common, _fill_workspace, _launch_key,
                            _validate_inputs)
 
 @dataclass(frozen=True)
@@ -358,7 +358,7 @@ def paged_decode_attention_cascade_into(
         except (AttributeError, TypeError):
             key = None  # an argument that is not a tensor: the full path raises the reference's message
         if key is not None and last[0] == key and (workspace is not None
-                                                   or not torch.cuda.is_current_stream_capturing()):
+                                                   or not _capturing(stream)):
             # the previous call's metadata and settings: only data pointers
             # change (a captured call's partials go to the graph's own memory)
             args, cas = last[1]

@@ -161,6 +161,12 @@ def _fill_append(args, append_k, append_v, slot_mapping):
     args.slot_mapping_stride = slot_mapping.stride(0)
 
 
+def _capturing(stream):
+    """Whether the current stream, of that handle, is being captured (the default stream, 0, never is: no question to
+    the runtime, 0.3 us)."""
+    return stream != 0 and torch.cuda.is_current_stream_capturing()
+
+
 class _SplitWorkspace:
     """fp32 split partials (plus zeroed arrival counters), reused across calls.
 
@@ -212,7 +218,7 @@ def _hold(held, key, ws):
 def _auto_workspace(q, num_kv_heads, num_splits, stream):
     num_seqs, num_q_heads, head_dim = q.shape
     floats = num_seqs * num_q_heads * num_splits * (head_dim + 2)
-    if torch.cuda.is_current_stream_capturing():
+    if _capturing(stream):
         return _SplitWorkspace(q.device, floats, 0).views(num_seqs, num_q_heads, num_splits, head_dim)
     counters = num_seqs * num_kv_heads * _lib.SPLIT_COUNTER_STRIDE
     key = (q.device.index, stream)
@@ -238,7 +244,7 @@ def _even_workspace(device, floats, stream):
     """fp32 scratch of one even-share call.  Looked up per call, and inside a graph capture allocated
     for that call alone: it then belongs to the graph's memory, so that no later call writes it between
     replays and none outlives it."""
-    if torch.cuda.is_current_stream_capturing():
+    if _capturing(stream):
         return torch.empty(floats, device=device, dtype=torch.float32)
     held = _EVEN_WORKSPACES.__dict__
     ws = held.get((device.index, stream))
@@ -271,12 +277,7 @@ def paged_decode_attention(
     from the cache when omitted (paged_decode.py:950-955).  ``ragged`` and
     ``kv_reuse``: see :func:`paged_decode_attention_into`.
     """
-    token_axis, _ = _layout_axes(kv_layout)
-    if block_size is None:
-        if k_cache.dim() != 4:
-            raise ValueError("k_cache must be a 4D tensor")
-        block_size = k_cache.shape[token_axis]
-    else:
+    if block_size is not None:
         block_size = int(block_size)
     out = torch.empty_like(q)
     return paged_decode_attention_into(
@@ -354,7 +355,7 @@ def paged_decode_attention_into(
         launch = last[1]
         if last[2] is not None:
             launch = last[2][_off_16(q, k_cache, v_cache, append_k, append_v)]
-        if launch is not None and launch[0].library_workspace and torch.cuda.is_current_stream_capturing():
+        if launch is not None and launch[0].library_workspace and _capturing(stream):
             launch = None  # a captured call's partials go to the graph's own memory
     if launch is not None:
         # the previous call's shapes, strides, dtypes, devices and settings:
