@@ -324,11 +324,12 @@ def paged_decode_attention_into(
     fuse the current token's cache write: the kernel stores it at the slot and
     attends to it from registers.  Mirrors paged_decode.py:972-1264.
 
-    Without a caller workspace the library plans the launch: large batches are
-    cut into equal shares of tokens whatever the rows' lengths are
-    (``fd_paged_decode_even``), smaller ones give every row the same number of
-    splits.  ``ragged=True`` (no counterpart in the reference) tells the second
-    plan that the batch's lengths vary widely: each row then gets splits in
+    Without a caller workspace the library plans the launch: batches large for
+    their block tables are cut into equal shares of tokens whatever the rows'
+    lengths are (``fd_paged_decode_even``, where ``fd_paged_decode_even_pays``
+    says so), others give every row the same number of splits.  ``ragged=True``
+    (no counterpart in the reference) says that the batch's lengths vary
+    widely: where equal shares do not pay, each row then gets splits in
     proportion to its length, counted on the device from ``seq_lens``
     (``balance_target`` of the C ABI).  It applies without fused append, and
     only where the batch leaves room in one round of workgroups; elsewhere it

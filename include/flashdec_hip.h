@@ -252,7 +252,7 @@ int fd_paged_decode_noalloc_prepare(fd_stream_t stream);
 
 /*
  * Shared-prefix (cascade) decode: the result of fd_paged_decode, with the
- * K/V of a prefix shared by a group of rows read once per 16 (member, query
+ * K/V of a prefix shared by a group of rows read once per chunk of (member, query
  * head) rows of the group.  No counterpart in the reference, which reads
  * every row's prefix separately (flashdec/kernels/paged_decode.py:330-543);
  * groups are the rows attached to one registered prefix of PagedKVCache
@@ -322,7 +322,8 @@ int fd_paged_decode_cascade(const fd_paged_decode_args* args, const fd_cascade_a
  * anything runs.  workspace: fp32 scratch, 16-byte aligned, at least
  * fd_paged_decode_even_floats(args) floats (0: the call is not one for this
  * function), with nothing in it that must be kept between calls; calls that
- * share one must be ordered on a stream.
+ * share one must be ordered on a stream.  Lengths that change under the launch
+ * leave rows wrong and nothing else.
  */
 int fd_paged_decode_even_floats(const fd_paged_decode_args* args);
 /* Whether the library would take fd_paged_decode_even for this call: 1 or 0
